@@ -62,6 +62,26 @@ std::vector<double> buffer_equilibrium(const std::vector<double> &kon, const std
     return ans;
 }
 
+// The compile-time species layout (Layout<LY>) matching the run-time one, or 0.
+int layout_id(const Params &p) {
+    if (p.ni != 1 || p.nb != 3 || p.nu != 3 || p.sl[0] || p.Db[0] == 0.0 || p.Db[1] == 0.0 || p.Db[2] != 0.0)
+        return 0;
+    for (int ly = 1; ly <= 2; ++ly) {
+        bool ok = true;
+        for (int b = 0; b < 3; ++b) {
+            const int bion = ly == 1 ? Layout<1>::bion[b] : Layout<2>::bion[b];
+            const int bbuf = ly == 1 ? Layout<1>::bbuf[b] : Layout<2>::bbuf[b];
+            const int bface = ly == 1 ? Layout<1>::bface[b] : Layout<2>::bface[b];
+            const int bslot = ly == 1 ? Layout<1>::bslot[b] : Layout<2>::bslot[b];
+            const int uf = ly == 1 ? Layout<1>::ufaces[b] : Layout<2>::ufaces[b];
+            ok = ok && p.bion[b] == bion && p.bbuf[b] == bbuf && p.bface[b] == bface && p.bslot[b] == bslot &&
+                 p.ufaces[b] == uf;
+        }
+        if (ok && p.n_grid == (ly == 1 ? 3 : 4) && p.n_face == (ly == 1 ? 1 : 0)) return ly;
+    }
+    return 0;
+}
+
 }  // namespace casim
 
 namespace {
@@ -116,6 +136,11 @@ void step_dispatch(CasimDyad *d, double dt) {
 }
 
 }  // namespace
+
+void CasimDyad::sync() {
+    HIPCK(hipStreamSynchronize(stream));
+    casim::resident_check(this);
+}
 
 void CasimDyad::launch_step(double dt) {
     if (precision == CASIM_FP64)
@@ -522,6 +547,7 @@ int casim_dyad_destroy(CasimDyad *d) {
     if (d->stream2) (void)hipStreamSynchronize(d->stream2);
     d->clear_graphs();
     casim::box_free(d);
+    casim::resident_free(d);
     void *ptrs[] = {d->g[0], d->g[1], d->f[0], d->f[1], d->d_off, d->d_node, d->d_type, d->d_perm, d->d_snode,
                     d->d_sperm, d->d_state, d->d_chans, d->d_rng, d->d_rng0, d->d_jump, d->d_mouths, d->d_jsr, d->d_sJ,
                     d->d_snap, d->d_pg, d->d_pjv, d->d_totals, d->d_rim_ions, d->d_rim_bound, d->d_eff, d->d_stats, d->Ch.trace};
@@ -634,7 +660,7 @@ int casim_dyad_update(CasimDyad *d, const double *rim_ions, const double *rim_bo
 namespace {
 void copy_out(CasimDyad *d, double *out, const double *src, size_t n) {
     HIPCK(hipMemcpyAsync(out, src, sizeof(double) * n, hipMemcpyDeviceToHost, d->stream));
-    HIPCK(hipStreamSynchronize(d->stream));
+    d->sync();
 }
 }  // namespace
 
@@ -806,6 +832,16 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
         REQUIRE(!d->box || k_steps % M == 0, CASIM_E_INVALID,
                 "with a cytosol box, k_steps must be a multiple of its substeps");
         d->use();
+        if (casim::resident_ok(d, k_steps)) {
+            for (int32_t left = k_steps; left > 0;) {
+                const int32_t kc = std::min(left, (int32_t)2048);
+                left -= kc;
+                casim::resident_steps(d, dt, kc);
+            }
+            d->launch_efflux();
+            d->launch_channels(CH_SNAPSHOT | CH_CURRENTS | CH_ACCUMULATE | CH_POOL_UPDATE, dt);
+            return;
+        }
         // One captured graph covers at most 2048 steps, a whole number of
         // box steps: a longer call replays several graphs, which gives the
         // results of one (each graph ends with the update that the next
@@ -1007,7 +1043,7 @@ int casim_dyad_synchronize(CasimDyad *d) {
     return guard([&] {
         REQUIRE(d, CASIM_E_INVALID, "null handle");
         d->use();
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 
@@ -1083,14 +1119,14 @@ void get_field_t(CasimDyad *d, int fi, double *out) {
         std::vector<T> h(N);
         HIPCK(hipMemcpyAsync(h.data(), (const T *)d->g[d->cur] + slot * N, sizeof(T) * N, hipMemcpyDeviceToHost,
                              d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         for (size_t i = 0; i < N; ++i) out[i] = (double)h[i];
     } else {
         const size_t F = (size_t)P.S * 2 * P.nFP;
         std::vector<T> h(F);
         HIPCK(hipMemcpyAsync(h.data(), (const T *)d->f[d->cur] + slot * F, sizeof(T) * F, hipMemcpyDeviceToHost,
                              d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         std::fill(out, out + N, 0.0);
         for (int s = 0; s < P.S; ++s)
             for (int xy = 0; xy < P.nFP; ++xy) {
@@ -1112,7 +1148,7 @@ void set_field_t(CasimDyad *d, int fi, const double *in) {
         for (size_t i = 0; i < N; ++i) h[i] = (T)in[i];
         for (int k = 0; k < 2; ++k)
             HIPCK(hipMemcpyAsync((T *)d->g[k] + slot * N, h.data(), sizeof(T) * N, hipMemcpyHostToDevice, d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     } else {
         const size_t F = (size_t)P.S * 2 * P.nFP;
         std::vector<T> h(F);
@@ -1123,7 +1159,7 @@ void set_field_t(CasimDyad *d, int fi, const double *in) {
             }
         for (int k = 0; k < 2; ++k)
             HIPCK(hipMemcpyAsync((T *)d->f[k] + slot * F, h.data(), sizeof(T) * F, hipMemcpyHostToDevice, d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     }
 }
 }  // namespace
@@ -1158,7 +1194,7 @@ int casim_dyad_get_channel_states(CasimDyad *d, int32_t *out) {
         d->use();
         std::vector<int> h(std::max(1, d->nch));
         HIPCK(hipMemcpyAsync(h.data(), d->d_state, sizeof(int) * d->nch, hipMemcpyDeviceToHost, d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         for (int s = 0; s < d->P.S; ++s) {
             int o = d->h_off[s], n = d->h_off[s + 1] - o;
             for (int j = 0; j < d->M; ++j) out[(size_t)s * d->M + j] = j < n ? h[o + j] : -1;
@@ -1180,7 +1216,7 @@ int casim_dyad_set_channel_states(CasimDyad *d, const int32_t *in) {
             }
         }
         HIPCK(hipMemcpyAsync(d->d_state, h.data(), sizeof(int) * d->nch, hipMemcpyHostToDevice, d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 
@@ -1190,7 +1226,7 @@ int casim_dyad_get_rng_states(CasimDyad *d, uint64_t *out) {
         d->use();
         std::vector<uint32_t> h((size_t)d->P.S * 6);
         HIPCK(hipMemcpyAsync(h.data(), d->d_rng, sizeof(uint32_t) * h.size(), hipMemcpyDeviceToHost, d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         for (size_t i = 0; i < h.size(); ++i) out[i] = h[i];
     });
 }
@@ -1205,7 +1241,7 @@ int casim_dyad_set_rng_states(CasimDyad *d, const uint64_t *in) {
             for (int i = 0; i < 6; ++i) h[6 * (size_t)s + i] = (uint32_t)in[6 * (size_t)s + i];
         }
         HIPCK(hipMemcpyAsync(d->d_rng, h.data(), sizeof(uint32_t) * h.size(), hipMemcpyHostToDevice, d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 
@@ -1265,7 +1301,7 @@ int casim_dyad_record_open_counts(CasimDyad *d, int32_t steps_per_bin, int32_t m
         REQUIRE(d, CASIM_E_INVALID, "null handle");
         REQUIRE(steps_per_bin >= 1 && max_bins >= 0, CASIM_E_INVALID, "steps_per_bin >= 1, max_bins >= 0");
         d->use();
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         if (d->Ch.trace) (void)hipFree(d->Ch.trace);
         d->Ch.trace = nullptr;
         d->Ch.trace_every = steps_per_bin;
@@ -1273,7 +1309,7 @@ int casim_dyad_record_open_counts(CasimDyad *d, int32_t steps_per_bin, int32_t m
         if (max_bins > 0) {
             HIPCK(hipMalloc(&d->Ch.trace, (size_t)max_bins * d->P.S));
             HIPCK(hipMemsetAsync(d->Ch.trace, 0xFF, (size_t)max_bins * d->P.S, d->stream));
-            HIPCK(hipStreamSynchronize(d->stream));
+            d->sync();
         }
         d->clear_graphs();
     });
@@ -1286,7 +1322,7 @@ int casim_dyad_get_open_counts(CasimDyad *d, uint8_t *out) {
         d->use();
         HIPCK(hipMemcpyAsync(out, d->Ch.trace, (size_t)d->Ch.trace_bins * d->P.S, hipMemcpyDeviceToHost,
                              d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 
@@ -1306,7 +1342,7 @@ int casim_dyad_set_split(CasimDyad *d, int32_t on) {
         REQUIRE(d, CASIM_E_INVALID, "null handle");
         REQUIRE(on == 0 || on == 1, CASIM_E_INVALID, "on must be 0 or 1");
         d->use();
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         if (d->split != (on != 0)) d->clear_graphs();
         d->split = on != 0;
     });

@@ -57,6 +57,7 @@ namespace casim {
 std::vector<double> buffer_equilibrium(const std::vector<double> &kon, const std::vector<double> &koff,
                                        const std::vector<double> &c, double total);
 struct CytoBox;  // 3D cytosol box around each site (cytosol_box.hip)
+struct Resident;  // plan and exchange buffers of the steps with the state on the chip (resident.hip)
 }  // namespace casim
 
 struct CasimDyad {
@@ -92,6 +93,8 @@ struct CasimDyad {
     int steps_per_pass = 2;   // 2: pairs of steps in one k_sweep2 pass where pair_ok()
     bool chan_small = false;  // the channel kernel's SheepCannell / one-ion instantiation applies
     casim::CytoBox *box = nullptr;  // cytosol box (null when not attached)
+    casim::Resident *res = nullptr;  // made by the first step that it can take
+    bool res_tried = false;
     // the sites and stream the pair and channel launchers work on (all sites
     // on `stream` unless casim_dyad_step splits the batch)
     int range_s0 = 0, range_n = -1;
@@ -111,6 +114,7 @@ struct CasimDyad {
     size_t face_elems() const { return (size_t)P.n_face * P.S * 2 * P.nFP; }
 
     void use() { HIPCK(hipSetDevice(dev)); }
+    void sync();  // the stream is idle and no step has failed
 
     void launch_step(double dt);
     bool pair_ok() const;
@@ -134,6 +138,18 @@ void sweep2_launch_f64_3d(CasimDyad *d, double dt);
 void sweep2_launch_f64_2d(CasimDyad *d, double dt);
 void sweep2_launch_f32_3d(CasimDyad *d, double dt);
 void sweep2_launch_f32_2d(CasimDyad *d, double dt);
+}  // namespace casim
+
+namespace casim {
+// Steps with the state on the chip (resident.hip).  resident_ok: the handle's
+// configuration has them (makes the plan at the first call); resident_steps: k
+// steps in one launch on the handle's stream, the buffers flipped once;
+// resident_check: throws when a launch gave up waiting.
+bool resident_ok(CasimDyad *d, int k_steps);
+void resident_steps(CasimDyad *d, double dt, int k);
+void resident_check(const CasimDyad *d);
+void resident_free(CasimDyad *d);
+int layout_id(const Params &p);  // compile-time species layout that fits, or 0 (casim_dyad.hip)
 }  // namespace casim
 
 namespace casim {

@@ -446,14 +446,11 @@ template <int LY> __device__ __forceinline__ double ly_total(const Params &p, in
 
 // Updated values of one interior node (DyadRDCPU.cpp:404-492): the
 // Laplacian of every diffusing field (x-neighbours from registers, y and z
-// from the LDS plane), the reactions with the free buffers seen by each
-// bound field, the channel current, the sarcolemmal factor at z = nz-1 (3D)
-// or everywhere (2D), the Euler step.  C0/Cm/Cp: the node and its x-1 / x+1
-// neighbours, every grid field; Fv: face values of the node.  The LDS plane
-// is node-major ([node][grid field]): Lc points at the node's first field,
-// its y-neighbours sit sy elements away and its z-neighbours zl, zr elements
-// away (the mirror image on the z-faces).  Writes the new grid values to G
-// (every grid field) and, at face nodes, the new face values to Fo.
+// from nbr), the reactions with the free buffers seen by each bound field,
+// the channel current, the sarcolemmal factor at z = nz-1 (3D) or everywhere
+// (2D), the Euler step.  C0/Cm/Cp: the node and its x-1 / x+1 neighbours,
+// every grid field; Fv: face values of the node.  Writes the new grid values
+// to G (every grid field) and, at face nodes, the new face values to Fo.
 //
 // The reference's terms, regrouped for FP64 issue: each Laplacian sums the
 // two neighbours of a direction first, ihx2 (u[x+1] + u[x-1]) + ihy2 (..)
@@ -462,23 +459,47 @@ template <int LY> __device__ __forceinline__ double ly_total(const Params &p, in
 // current) for an ion and D lap - R1 for a bound field (7 + 2 operations
 // per diffusing field where the reference's order takes 10 + 3).  The
 // values differ from the reference's order by rounding only.
-template <typename T, int DIM, int NI, int NB, int NG, int NF, int LY, int LI_ = NI ? NI : MAXI>
+//
+// nbr gives the y- and z-neighbours' values of a field (z: the mirror image on
+// the z-faces): LdsNbr reads them from a node-major LDS plane ([node][grid
+// field]), its y-neighbours sy elements away and its z-neighbours dl, dr;
+// RegNbr holds them in registers, for a kernel that updates several planes in
+// a row.
+template <typename T>
+struct LdsNbr {
+    static constexpr bool regs = false;
+    const T *L;  // the node's first field
+    int sy, dl, dr;
+    __device__ __forceinline__ T yl(int g) const { return L[g - sy]; }
+    __device__ __forceinline__ T yr(int g) const { return L[g + sy]; }
+    __device__ __forceinline__ T zl(int g) const { return L[g + dl]; }
+    __device__ __forceinline__ T zr(int g) const { return L[g + dr]; }
+};
+template <typename T, int NG>
+struct RegNbr {
+    static constexpr bool regs = true;
+    T v[4][NG];
+    __device__ __forceinline__ T yl(int g) const { return v[0][g]; }
+    __device__ __forceinline__ T yr(int g) const { return v[1][g]; }
+    __device__ __forceinline__ T zl(int g) const { return v[2][g]; }
+    __device__ __forceinline__ T zr(int g) const { return v[3][g]; }
+};
+template <typename T, int DIM, int NI, int NB, int NG, int NF, int LY, typename Nbr, int LI_ = NI ? NI : MAXI>
 __device__ __forceinline__ void node_update(const Params &p, const T *Cm, const T (&C0)[NG],
-                                            const T (&Cp)[NG], const T *Lc, int sy, int zl, int zr, int z,
+                                            const T (&Cp)[NG], const Nbr &nbr, int z,
                                             bool face, const T (&Fv)[NF], const T (&J)[LI_], T dt, T ihx2, T ihy2, T ihz2,
                                             T (&G)[NG], T (&Fo)[NF]) {
     constexpr int LI = NI ? NI : MAXI;
     constexpr int LB = NB ? NB : MAXB;
     const T cc = (T)p.cc;
     T Cv[LI], lC[LI], Bv[LB], lB[LB];
-    const T *Lyl = Lc - sy, *Lyr = Lc + sy, *Lzl = Lc + zl, *Lzr = Lc + zr;
 #pragma unroll
     for (int j = 0; j < LI; ++j) {
         if (!NI && j >= p.ni) break;
         const T vc = C0[j];
         Cv[j] = vc;
-        T lap = (Cp[j] + Cm[j]) * ihx2 + (Lyr[j] + Lyl[j]) * ihy2;
-        if (DIM == 3) lap = lap + (Lzr[j] + Lzl[j]) * ihz2;
+        T lap = (Cp[j] + Cm[j]) * ihx2 + (nbr.yr(j) + nbr.yl(j)) * ihy2;
+        if (DIM == 3) lap = lap + (nbr.zr(j) + nbr.zl(j)) * ihz2;
         lC[j] = lap - cc * vc;
     }
 #pragma unroll
@@ -503,8 +524,8 @@ __device__ __forceinline__ void node_update(const Params &p, const T *Cm, const 
                 }
             Bv[b] = vc;
             if (ly_mobile<LY>(p, b)) {
-                T lap = (cxr + cxl) * ihx2 + (Lyr[g] + Lyl[g]) * ihy2;
-                if (DIM == 3) lap = lap + (Lzr[g] + Lzl[g]) * ihz2;
+                T lap = (cxr + cxl) * ihx2 + (nbr.yr(g) + nbr.yl(g)) * ihy2;
+                if (DIM == 3) lap = lap + (nbr.zr(g) + nbr.zl(g)) * ihz2;
                 lB[b] = lap - cc * vc;
             }
         }
@@ -540,9 +561,23 @@ __device__ __forceinline__ void node_update(const Params &p, const T *Cm, const 
         const T R1 = (T)p.koff[b] * Bv[b] - (T)p.kon[b] * cj * frb[b];
         eB[b] = ly_mobile<LY>(p, b) ? (T)p.Db[b] * lB[b] - R1 : -R1;
         const bool on = !ly_bface<LY>(p, b) || face;
+        T add = R1;
+        if constexpr (Nbr::regs) {
+            // a select, not a branch on the face lanes: a kernel that updates
+            // several planes in a row would otherwise gather all of them
+            // before the branch and hold their neighbours in registers
+            if (ly_bface<LY>(p, b)) {
+                asm("" : "+v"(add));
+                add = on ? add : (T)-0.0;  // x + -0 == x
+            }
 #pragma unroll
-        for (int jj = 0; jj < LI; ++jj)
-            if (jj == j && on) Rr[jj] += R1;
+            for (int jj = 0; jj < LI; ++jj)
+                if (jj == j) Rr[jj] += add;
+        } else {
+#pragma unroll
+            for (int jj = 0; jj < LI; ++jj)
+                if (jj == j && on) Rr[jj] += R1;
+        }
     }
 #pragma unroll
     for (int j = 0; j < LI; ++j) {
@@ -728,8 +763,8 @@ __global__ __launch_bounds__(512) void k_sweep(const T *__restrict__ gin, T *__r
             const int z = DIM == 3 ? c % p.nz : 0;
             T G[NG], Fo[NF];
             if (ps.inner[k]) {
-                node_update<T, DIM, NI, NB, NG, NF, LY>(p, R[0][k], R[1][k], R[2][k], L + c * ng, p.nz * ng,
-                                                    ps.zl[k] * ng, ps.zr[k] * ng, z,
+                const LdsNbr<T> nbr{L + c * ng, p.nz * ng, ps.zl[k] * ng, ps.zr[k] * ng};
+                node_update<T, DIM, NI, NB, NG, NF, LY>(p, R[0][k], R[1][k], R[2][k], nbr, z,
                                                     ps.fz[k] >= 0, F[0][k], J[k], dt, ihx2, ihy2, ihz2, G, Fo);
             } else {
 #pragma unroll
@@ -937,9 +972,8 @@ __global__ __launch_bounds__(512) CASIM_SWEEP2_ATTR void k_sweep2(const T *__res
                     const int z = DIM == 3 ? c % p.nz : 0;
                     const T *cm = R[0][k];
                     if constexpr (LPREV) cm = LA + (size_t)((x - 1) & 1) * ng * P + c * ng;
-                    node_update<T, DIM, NI, NB, NG, NF, LY>(p, cm, R[1][k], R[2][k], La + c * ng, p.nz * ng,
-                                                        ps.zl[k] * ng, ps.zr[k] * ng,
-                                                        z, (fl[k] & 4) != 0, F[0][k], J[k], dt, ihx2, ihy2, ihz2,
+                    const LdsNbr<T> nbr{La + c * ng, p.nz * ng, ps.zl[k] * ng, ps.zr[k] * ng};
+                    node_update<T, DIM, NI, NB, NG, NF, LY>(p, cm, R[1][k], R[2][k], nbr, z, (fl[k] & 4) != 0, F[0][k], J[k], dt, ihx2, ihy2, ihz2,
                                                         A[2][k], FA[1][k]);
                 } else {
 #pragma unroll
@@ -1028,8 +1062,8 @@ __global__ __launch_bounds__(512) CASIM_SWEEP2_ATTR void k_sweep2(const T *__res
                 if (fl[k] & 2) {
                     const T *cm = A[0][k];
                     if constexpr (LPREV) cm = LB2 + (size_t)(x & 1) * ng * P + c * ng;  // plane x-2
-                    node_update<T, DIM, NI, NB, NG, NF, LY>(p, cm, A[1][k], A[2][k], Lb + c * ng, p.nz * ng,
-                                                        ps.zl[k] * ng, ps.zr[k] * ng, z, (fl[k] & 4) != 0,
+                    const LdsNbr<T> nbr{Lb + c * ng, p.nz * ng, ps.zl[k] * ng, ps.zr[k] * ng};
+                    node_update<T, DIM, NI, NB, NG, NF, LY>(p, cm, A[1][k], A[2][k], nbr, z, (fl[k] & 4) != 0,
                                                         FA[0][k], J[k], dt, ihx2, ihy2, ihz2, G, Fo);
                 } else {
 #pragma unroll

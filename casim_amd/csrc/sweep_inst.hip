@@ -37,26 +37,6 @@ void sweep_slots(CasimDyad *d, double dt) {
     return sweep_launch<T, DIM, NI, NB, NG, NF, LY, 4, 1>(d, dt);
 }
 
-// The compile-time species layout (Layout<LY>) matching the run-time one, or 0.
-int layout_id(const Params &p) {
-    if (p.ni != 1 || p.nb != 3 || p.nu != 3 || p.sl[0] || p.Db[0] == 0.0 || p.Db[1] == 0.0 || p.Db[2] != 0.0)
-        return 0;
-    for (int ly = 1; ly <= 2; ++ly) {
-        bool ok = true;
-        for (int b = 0; b < 3; ++b) {
-            const int bion = ly == 1 ? Layout<1>::bion[b] : Layout<2>::bion[b];
-            const int bbuf = ly == 1 ? Layout<1>::bbuf[b] : Layout<2>::bbuf[b];
-            const int bface = ly == 1 ? Layout<1>::bface[b] : Layout<2>::bface[b];
-            const int bslot = ly == 1 ? Layout<1>::bslot[b] : Layout<2>::bslot[b];
-            const int uf = ly == 1 ? Layout<1>::ufaces[b] : Layout<2>::ufaces[b];
-            ok = ok && p.bion[b] == bion && p.bbuf[b] == bbuf && p.bface[b] == bface && p.bslot[b] == bslot &&
-                 p.ufaces[b] == uf;
-        }
-        if (ok && p.n_grid == (ly == 1 ? 3 : 4) && p.n_face == (ly == 1 ? 1 : 0)) return ly;
-    }
-    return 0;
-}
-
 template <typename T, int DIM, int NI, int NB, int NG, int NF, int LY, int SL, bool RING>
 void sweep2_ring(CasimDyad *d, double dt) {
     const Params &p = d->P;

@@ -236,14 +236,19 @@ int casim_dyad_run_mc(CasimDyad *d, double dt, int32_t site);
  * last casim_dyad_update call.  The launches are captured once into a HIP
  * graph per (step count, dt) and replayed; one graph holds at most 2048 steps
  * (with a cytosol box, the most whole box steps below that), so a longer call
- * replays several graphs, with the results of one call.
+ * replays several graphs, with the results of one call.  3D one-ion layouts
+ * without a cytosol pool or box keep the state on the chip over the steps of a
+ * call instead, where the number of steps pays for it; results do not depend
+ * on that either.  casim_dyad_set_steps_per_pass(d, 1) selects the sweeps.
  */
 int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps);
 
 /* The same k_steps as casim_dyad_step, launched eagerly (no graph) with a
  * HIP event pair around every kernel on the handle's stream.  kernel_ms[0]
  * receives the summed duration of the state-sweep kernels, kernel_ms[1] that
- * of the channel kernels.  For measurement; results equal casim_dyad_step's. */
+ * of the channel kernels.  For measurement of the sweep kernels, which it runs
+ * also where casim_dyad_step keeps the state on the chip; results equal
+ * casim_dyad_step's. */
 int casim_dyad_step_profiled(CasimDyad *d, double dt, int32_t k_steps, double kernel_ms[2]);
 
 /* Block until the handle's stream is idle. */
