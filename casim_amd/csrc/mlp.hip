@@ -125,6 +125,15 @@ __global__ __launch_bounds__(256) void k_gemm(const uint16_t *__restrict__ A, in
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.f / (1.f + __expf(-z)); }
 
+// f2bf of four values by the conversion instruction (two values each, the same
+// rounding)
+__device__ __forceinline__ void f2bf4(const float (&f)[4], uint16_t (&h)[4]) {
+    __bf16 b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = (__bf16)f[i];
+    std::memcpy(h, b, sizeof h);
+}
+
 // Z += b (per column); H = bf16(SiLU(Z)) or bf16(Z) for the last layer.
 __global__ void k_bias_act(float *__restrict__ Z, const float *__restrict__ b, uint16_t *__restrict__ H, int rows,
                            int cols, int act) {
@@ -135,19 +144,29 @@ __global__ void k_bias_act(float *__restrict__ Z, const float *__restrict__ b, u
     if (H) H[i] = f2bf(act ? z * sigmoidf_(z) : z);
 }
 
-// Inference of one ensemble member for IMR rows per workgroup, every layer in
+// Inference of one ensemble member for 16 RT rows per workgroup, every layer in
 // one launch: the normalised BF16 input (k_gather's arithmetic), each hidden
 // layer as BF16 MFMA products with FP32 accumulation (k_gemm's operand layout
 // and k order), bias, SiLU and BF16 rounding (k_bias_act's), and the linear
-// output, with the activations in LDS.  The weights come transposed and
-// zero-padded ([n][k], k_wt) so a lane's eight k-values of an MFMA operand are
-// one 16-byte load.  Per output element the operations and their order are
-// those of k_gather + k_gemm + k_bias_act, so the outputs are the same bits.
-// Grid: (row tiles, members); sixteen waves, wave w computes the 16 columns
-// 16w .. +15 of a layer, and a lane loads all of the layer's k-blocks of its
-// weight row at once (at most IMAXW / 32 = 8) while the layer before runs:
-// with few rows a workgroup is a latency chain of layers.
+// output, with the activations in LDS.  The weights come zero-padded in the
+// order of MFMA operands (k_wt).  Per output element the operations and their
+// order are those of k_gather + k_gemm + k_bias_act, so the outputs are the
+// same bits.  Grid: (row tiles, members).
+//
+// Few rows: sixteen waves with 16 columns each, 32 rows.  A workgroup is a
+// latency chain of layers, so a lane has all of the next layer's weights on
+// their way while a layer runs.  Many rows: eight waves with 32 columns each, 64
+// rows, two workgroups per CU.  The weights are then read half as often and the
+// rows' operands from LDS feed two products; what bounds it is the SiLU, about
+// 25 vector operations per activation.  Times in us for five members of width
+// 256, depth 4 (before: weights in plain rows, 32 rows per workgroup):
+//   rows        512   2048   4096   8192   16384   55003
+//   before       -      -      -      -      195     658
+//   32 rows      17     29     42     66     126     424
+//   64 rows      26     28     39     55      86     276
+// so 64 rows from INFER_BIG workgroups on, one per CU.
 constexpr int IMR = 32, IMAXW = 256, IPADK = 8, IMAXM = 8, IMAXL = 8, IWAVES = IMAXW / 16;
+constexpr size_t INFER_BIG = 256;
 struct InferArgs {
     const uint16_t *wt[IMAXM];  // member's transposed weights
     const float *p[IMAXM];      // member's FP32 parameters (biases at boff)
@@ -156,37 +175,63 @@ struct InferArgs {
     const float *mean, *istd;
 };
 
-__global__ void k_wt(const uint16_t *__restrict__ W, uint16_t *__restrict__ WT, int fin, int fout, int kp, int np) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)np * kp) return;
-    const int n = (int)(i / kp), k = (int)(i % kp);
-    WT[i] = (n < fout && k < fin) ? W[(size_t)k * fout + n] : (uint16_t)0;
+// Place of element (n, k) of a [n][k] operand with nk blocks of 32 in k, in the
+// order in which an MFMA operand's lanes hold it: blocks of 16 n and 32 k, in
+// them lane by lane eight consecutive k.  A wave's load of a block is 1 KiB in
+// a row; with plain rows it is 16 half lines, and L2 moves each line twice.
+__host__ __device__ inline int frag_at(int n, int k, int nk) {
+    return (((n >> 4) * nk + (k >> 5)) << 9) + (((k >> 3 & 3) << 4 | (n & 15)) << 3) + (k & 7);
 }
 
-__global__ __launch_bounds__(64 * IWAVES) void k_mlp_infer(const float *__restrict__ X, int rows,
-                                                            float *__restrict__ out, int ostride, InferArgs a) {
-    __shared__ __attribute__((aligned(16))) uint16_t H[2][IMR][IMAXW + IPADK];
-    const int m0 = blockIdx.x * IMR, e = blockIdx.y;
+// Every layer's and member's W [fin][fout] -> zero-padded operands of the
+// forward product (n over fout, k over fin) and of the product with W^T of the
+// backward pass (n over fin, k over fout).  Grid: (elements, 2 layers, members).
+struct WtArgs {
+    const uint16_t *pb[IMAXM];
+    uint16_t *wt[IMAXM];
+    int woff[IMAXL], fin[IMAXL], fout[IMAXL], off[2 * IMAXL];  // off: operand of layer g / 2, backward if g % 2
+};
+__global__ void k_wt(const WtArgs a) {
+    const int g = blockIdx.y, L = g >> 1, back = g & 1, e = blockIdx.z;
+    const int nn = back ? a.fin[L] : a.fout[L], nk = back ? a.fout[L] : a.fin[L];
+    const int kp = (nk + 31) & ~31, np = (nn + 15) & ~15;
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= np * kp) return;
+    const int n = i / kp, k = i - n * kp;
+    uint16_t v = 0;
+    if (n < nn && k < nk) v = a.pb[e][a.woff[L] + (back ? n * a.fout[L] + k : k * a.fout[L] + n)];
+    a.wt[e][a.off[g] + frag_at(n, k, kp >> 5)] = v;
+}
+
+template <int CT, int RT>
+__global__ __launch_bounds__(64 * IWAVES / CT, 4) void k_mlp_infer(const float *__restrict__ X, int rows,
+                                                                   float *__restrict__ out, int ostride, InferArgs a) {
+    constexpr int R = 16 * RT, NT = 64 * IWAVES / CT;
+    __shared__ __attribute__((aligned(16))) uint16_t H[2][R][IMAXW + IPADK];
+    const int m0 = blockIdx.x * R, e = blockIdx.y;
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
     const uint16_t *wt = a.wt[e];
     const float *pe = a.p[e];
-    // every k-block of the lane's weight row for layer L, and its bias, issued
-    // together (blocks past the layer's K repeat its last one, columns past
-    // its width the last row; neither is used)
-    auto fetch = [&](int L, bf16x8_t (&b)[IMAXW / 32], float &bias) {
-        const int K = a.kp[L], N = a.fout[L], NP = (N + 15) & ~15, nk = K >> 5;
-        const int col = min(w * 16 + (l & 15), NP - 1);
-        const uint16_t *wrow = wt + a.wtoff[L] + (size_t)col * K + (l >> 4) * 8;
+    // every k-block of the wave's columns for layer L, and their biases, issued
+    // together (blocks past the layer's K repeat its last one, columns past its
+    // width its last tile; neither is used)
+    auto fetch = [&](int L, bf16x8_t (&b)[CT][IMAXW / 32], float (&bias)[CT]) {
+        const int N = a.fout[L], nk = a.kp[L] >> 5, nt = (N + 15) >> 4;
 #pragma unroll
-        for (int kb = 0; kb < IMAXW / 32; ++kb)
-            b[kb] = *reinterpret_cast<const bf16x8_t *>(wrow + 32 * (kb < nk ? kb : nk - 1));
-        bias = pe[a.boff[L] + min(col, N - 1)];
+        for (int c = 0; c < CT; ++c) {
+            const int ct = min(w * CT + c, nt - 1);
+            const uint16_t *wf = wt + a.wtoff[L] + ((ct * nk) << 9) + l * 8;
+#pragma unroll
+            for (int kb = 0; kb < IMAXW / 32; ++kb)
+                b[c][kb] = *reinterpret_cast<const bf16x8_t *>(wf + ((kb < nk ? kb : nk - 1) << 9));
+            bias[c] = pe[a.boff[L] + min(ct * 16 + (l & 15), N - 1)];
+        }
     };
-    bf16x8_t bw[IMAXW / 32], bn[IMAXW / 32];
-    float bias, bias_n;
+    bf16x8_t bw[CT][IMAXW / 32], bn[CT][IMAXW / 32];
+    float bias[CT], bias_n[CT];
     fetch(0, bw, bias);  // in flight while the input is staged
     const int kp0 = a.kp[0];
-    for (int i = t; i < IMR * kp0; i += 64 * IWAVES) {
+    for (int i = t; i < R * kp0; i += NT) {
         const int r = i / kp0, f = i - r * kp0;
         uint16_t v = 0;
         if (m0 + r < rows && f < a.n_in) v = f2bf((X[(size_t)(m0 + r) * a.n_in + f] - a.mean[f]) * a.istd[f]);
@@ -194,47 +239,76 @@ __global__ __launch_bounds__(64 * IWAVES) void k_mlp_infer(const float *__restri
     }
     __syncthreads();
     for (int L = 0; L < a.nl; ++L) {
-        const int src = L & 1, K = a.kp[L], N = a.fout[L], NP = (N + 15) & ~15;
+        const int src = L & 1, N = a.fout[L], nk = a.kp[L] >> 5;
         const bool last = L == a.nl - 1;
-        const int n0 = w * 16;
         // the next layer's weights are in flight during this layer (the last
         // layer fetches itself again, so that the count of loads in flight is
-        // the same every layer)
-        fetch(last ? L : L + 1, bn, bias_n);
-        if (n0 < NP) {
-            const int nk = K >> 5;  // 32-wide k-blocks, at most 8
-            f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+        // the same every layer); a wave with two column tiles has the registers
+        // for them only once its products are done
+        if (CT == 1) fetch(last ? L : L + 1, bn, bias_n);
+        f32x4_t acc[CT][RT];
+        const bool on = w * CT * 16 < N;
+        if (on) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int i = 0; i < RT; ++i) acc[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kb = 0; kb < IMAXW / 32; ++kb) {
                 if (kb >= nk) break;
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
+                for (int i = 0; i < RT; ++i) {
                     const bf16x8_t av =
                         *reinterpret_cast<const bf16x8_t *>(&H[src][i * 16 + (l & 15)][32 * kb + (l >> 4) * 8]);
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[kb], acc[i], 0, 0, 0);
+#pragma unroll
+                    for (int c = 0; c < CT; ++c)
+                        acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bw[c][kb], acc[c][i], 0, 0, 0);
                 }
             }
-            const int col = n0 + (l & 15);
-            if (col < N) {
+        }
+        float b0[CT];
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+        for (int c = 0; c < CT; ++c) b0[c] = bias[c];
+        if (CT > 1 && !last) fetch(L + 1, bw, bias);
+        if (on) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int row = i * 16 + (l >> 4) * 4 + r;
-                        const float z = acc[i][r] + bias;
-                        if (last) {
-                            if (m0 + row < rows) out[(size_t)e * ostride + m0 + row] = z;
-                        } else {
-                            H[src ^ 1][row][col] = f2bf(z * sigmoidf_(z));
-                        }
+            for (int c = 0; c < CT; ++c) {
+                const int col = (w * CT + c) * 16 + (l & 15);
+                if (col >= N) break;
+#pragma unroll
+                for (int i = 0; i < RT; ++i) {
+                    const int row = i * 16 + (l >> 4) * 4;
+                    float z[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) z[r] = acc[c][i][r] + b0[c];
+                    if (last) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (m0 + row + r < rows) out[(size_t)e * ostride + m0 + row + r] = z[r];
+                    } else {
+                        uint16_t h[4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) z[r] *= sigmoidf_(z[r]);
+                        f2bf4(z, h);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) H[src ^ 1][row + r][col] = h[r];
                     }
+                }
             }
         }
         __syncthreads();
+        if (CT == 1) {
 #pragma unroll
-        for (int kb = 0; kb < IMAXW / 32; ++kb) bw[kb] = bn[kb];
-        bias = bias_n;
+            for (int kb = 0; kb < IMAXW / 32; ++kb) bw[0][kb] = bn[0][kb];
+            bias[0] = bias_n[0];
+        }
     }
+}
+
+// dH * SiLU'(z)
+__device__ __forceinline__ float silu_back(float dH, float z) {
+    const float s = sigmoidf_(z);
+    return dH * s * (1.f + z * (1.f - s));
 }
 
 // dZ = dH * SiLU'(Z), kept in FP32 (bias gradient) and BF16 (GEMM operand).
@@ -242,9 +316,7 @@ __global__ void k_silu_back(const float *__restrict__ dH, const float *__restric
                             uint16_t *__restrict__ dZb, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float z = Z[i];
-    const float s = sigmoidf_(z);
-    const float d = dH[i] * s * (1.f + z * (1.f - s));
+    const float d = silu_back(dH[i], Z[i]);
     dZ[i] = d;
     dZb[i] = f2bf(d);
 }
@@ -254,6 +326,7 @@ __global__ void k_colsum(const float *__restrict__ X, float *__restrict__ out, i
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= cols) return;
     float s = 0.f;
+#pragma unroll 16
     for (int r = 0; r < rows; ++r) s += X[(size_t)r * cols + c];
     out[c] = s;
 }
@@ -282,20 +355,362 @@ __global__ void k_mse(const float *__restrict__ pred, const float *__restrict__ 
     sq[i] = e * e;
 }
 
-// Adam on FP32 master weights; refresh the BF16 copy.
+// Adam on one FP32 master weight w with moments m and v and gradient g; the
+// fused operations are written out, so that every kernel rounds alike.
+struct AdamArgs {
+    float lr, b1, b2, eps;
+};
+__device__ __forceinline__ void adam_update(float &w, float &m, float &v, float g, const AdamArgs &a, float c1, float c2) {
+#pragma clang fp contract(off)
+    m = __builtin_fmaf(1.f - a.b1, g, a.b1 * m);
+    v = __builtin_fmaf(g, (1.f - a.b2) * g, a.b2 * v);
+    w = w - a.lr * (m / c1) / (sqrtf(v / c2) + a.eps);
+}
+// ... with a refresh of the BF16 copy.
 __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
-                       float *__restrict__ v, uint16_t *__restrict__ pb, size_t n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
+                       float *__restrict__ v, uint16_t *__restrict__ pb, size_t n, AdamArgs a, float c1, float c2) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+    float w = p[i], mi = m[i], vi = v[i];
+    adam_update(w, mi, vi, g[i], a, c1, c2);
     m[i] = mi;
     v[i] = vi;
-    const float w = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     p[i] = w;
     pb[i] = f2bf(w);
+}
+
+// ---------------------------------------------------------------------------
+// A training step of every member in two launches.
+//
+// k_train_rows: forward, loss and the chain of dZ down the layers for IMR rows
+// per workgroup, which need nothing of any other row: the activations of a
+// tile stay in LDS as in k_mlp_infer.  It leaves what the weight gradients
+// contract over the batch, the layers' inputs X and dZ in BF16 as operands with
+// the batch as k (frag_at's order: a wave's 32 x 16 results are one block of
+// 1 KiB), and dZ in FP32, rows first, for the bias gradients.
+// k_train_weights: a 64 x 64 tile of a layer's dW = X^T dZ, or the column sums
+// of dZ for 256 biases, and Adam on what it formed: weights, moments, the BF16
+// copy and its transposed copy for the next forward pass.
+//
+// Per element the operations and their order are those of k_gather, k_gemm,
+// k_bias_act, k_mse, k_silu_back, k_colsum and k_adam (k ascending in blocks of
+// 32, column sums from the first row on), which a layer at a time and a member
+// at a time took 34 launches per member and step, most of the time in k_colsum
+// (187 us for 256 columns: a chain of dependent loads).
+struct TrainArgs {
+    uint16_t *wt[IMAXM];
+    float *p[IMAXM], *am[IMAXM], *av[IMAXM];
+    float c1[IMAXM], c2[IMAXM];
+    int wtoff[2 * IMAXL], woff[IMAXL], boff[IMAXL], kp[IMAXL], fin[IMAXL], fout[IMAXL];
+    int xt0[IMAXL], zt0[IMAXL];    // first tile of 16 columns of a layer's X and dZ operands
+    int xtiles, ztiles;            // tiles of a member's operands, `tiles` blocks of 32 batch rows each
+    int zcol[IMAXL], zcols;        // first column of a layer's dZ in FP32; columns of a member
+    int tile0[IMAXL + 1];          // first weight tile of a layer
+    int mg, nsum;                  // members; workgroups that form a member's column sums, its first ones
+    int nl, n_in, B, tiles;        // tiles: of IMR rows
+    const float *mean, *istd, *X, *Y;
+    const int *perm;  // [members][rows] + the batch's first row
+    int64_t rows;
+    float ym, yis;
+    uint16_t *XT, *DZT;
+    float *DZ, *Z, *sq;  // sq: [members][sqn] + the batch's first row
+    int64_t sqn;
+    AdamArgs adam;
+};
+
+// prediction less the normalised target, which k_gather rounds and stores
+__device__ __forceinline__ float target_error(float pred, float y, float ym, float yis) {
+#pragma clang fp contract(off)
+    const float t = (y - ym) * yis;
+    return pred - t;
+}
+
+// This workgroup's unit of `units`, dealt so that the workgroups of a chiplet
+// (block index modulo 8) take units in a row, the same member's and layer's:
+// what they share is then read into one L2.  -1: none.
+__device__ __forceinline__ int chiplet_unit(int units) {
+    const int per = (units + 7) / 8, u = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    return (int)(blockIdx.x >> 3) < per && u < units ? u : -1;
+}
+__host__ inline unsigned chiplet_grid(int units) { return (unsigned)(units + 7) / 8 * 8; }
+
+__device__ __forceinline__ uint64_t pack4(const uint16_t (&h)[4]) {
+    return (uint64_t)h[0] | (uint64_t)h[1] << 16 | (uint64_t)h[2] << 32 | (uint64_t)h[3] << 48;
+}
+
+// Latency-bound: 32 workgroups per member at 1024 rows, each a chain of 2 depth
+// + 1 layers of eight MFMA pairs per wave between barriers, weights fetched a
+// layer ahead.  Five members, 1024 rows, width 256, depth 4: 34 us; 49 with the
+// weights in plain rows.
+__global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
+    __shared__ __attribute__((aligned(16))) uint16_t H[2][IMR][IMAXW + IPADK];
+    __shared__ int src[IMR];
+    const int unit = chiplet_unit(a.tiles * a.mg);
+    if (unit < 0) return;
+    const int e = unit / a.tiles, tile = unit - e * a.tiles, m0 = tile * IMR;
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
+    const uint16_t *wt = a.wt[e];
+    const float *pe = a.p[e];
+    uint16_t *XT = a.XT + ((size_t)e * a.xtiles * a.tiles + tile) * 512;  // block `tile` of column tile 0
+    uint16_t *DZT = a.DZT + ((size_t)e * a.ztiles * a.tiles + tile) * 512;
+    float *DZ = a.DZ + ((size_t)e * a.tiles * IMR + m0) * a.zcols;
+    const size_t ts = (size_t)a.tiles * 512;  // one column tile
+    f32x4_t *Z = reinterpret_cast<f32x4_t *>(a.Z) + ((size_t)e * a.tiles + tile) * (a.nl - 1) * IWAVES * 128 + w * 128 + l;
+    const int n0 = w * 16, c = n0 + (l & 15), kq = (l >> 4) * 8, rq = (l >> 4) * 4;
+    // the wave's k-blocks of an operand (blocks past K repeat the last one,
+    // columns past the width the last tile; neither is used)
+    auto weights = [&](int g, int N, int K, bf16x8_t(&b)[IMAXW / 32]) {
+        const int nk = (K + 31) >> 5;
+        const uint16_t *wf = wt + a.wtoff[g] + ((min(w, (N - 1) >> 4) * nk) << 9) + l * 8;
+#pragma unroll
+        for (int kb = 0; kb < IMAXW / 32; ++kb) b[kb] = *reinterpret_cast<const bf16x8_t *>(wf + ((kb < nk ? kb : nk - 1) << 9));
+    };
+    auto forward_w = [&](int L, bf16x8_t(&b)[IMAXW / 32], float &bias) {
+        weights(2 * L, a.fout[L], a.fin[L], b);
+        bias = pe[a.boff[L] + min(c, a.fout[L] - 1)];
+    };
+    auto backward_w = [&](int L, bf16x8_t(&b)[IMAXW / 32]) { weights(2 * L + 1, a.fin[L], a.fout[L], b); };
+    auto product = [&](int from, int nk, const bf16x8_t(&b)[IMAXW / 32], f32x4_t(&acc)[2]) {
+        acc[0] = acc[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < IMAXW / 32; ++kb) {
+            if (kb >= nk) break;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const bf16x8_t av = *reinterpret_cast<const bf16x8_t *>(&H[from][i * 16 + (l & 15)][32 * kb + kq]);
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b[kb], acc[i], 0, 0, 0);
+            }
+        }
+    };
+    bf16x8_t bw[IMAXW / 32], bn[IMAXW / 32];
+    float bias, bias_n = 0.f;
+    forward_w(0, bw, bias);
+    if (t < IMR) src[t] = m0 + t < a.B ? a.perm[(size_t)e * a.rows + m0 + t] : -1;
+    __syncthreads();
+    const int kp0 = a.kp[0];
+    for (int i = t; i < IMR * kp0; i += 64 * IWAVES) {
+        const int r = i / kp0, f = i - r * kp0;
+        uint16_t v = 0;
+        if (src[r] >= 0 && f < a.n_in) v = f2bf((a.X[(size_t)src[r] * a.n_in + f] - a.mean[f]) * a.istd[f]);
+        H[0][r][f] = v;
+    }
+    __syncthreads();
+    for (int i = t; i < a.n_in * (IMR / 4); i += 64 * IWAVES) {
+        const int f = i / (IMR / 4), r = i % (IMR / 4) * 4;
+        const uint16_t h[4] = {H[0][r][f], H[0][r + 1][f], H[0][r + 2][f], H[0][r + 3][f]};
+        *reinterpret_cast<uint64_t *>(XT + (a.xt0[0] + (f >> 4)) * ts + frag_at(f & 15, r, 1)) = pack4(h);
+    }
+    const int last = a.nl - 1;
+    for (int L = 0; L < last; ++L) {
+        forward_w(L + 1, bn, bias_n);
+        if (n0 < a.fout[L]) {
+            f32x4_t acc[2];
+            product(L & 1, a.kp[L] >> 5, bw, acc);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                f32x4_t zz;
+                float f[4];
+                uint16_t h[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float z = acc[i][r] + bias;
+                    zz[r] = z;
+                    f[r] = z * sigmoidf_(z);
+                }
+                f2bf4(f, h);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = i * 16 + rq + r;
+                    H[(L & 1) ^ 1][row][c] = h[r];
+                    if (m0 + row >= a.B) h[r] = 0;
+                }
+                Z[(L * IWAVES * 2 + i) * 64] = zz;
+                *reinterpret_cast<uint64_t *>(XT + (a.xt0[L + 1] + w) * ts + frag_at(l & 15, i * 16 + rq, 1)) = pack4(h);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kb = 0; kb < IMAXW / 32; ++kb) bw[kb] = bn[kb];
+        bias = bias_n;
+    }
+    // output column, loss and its derivative; the other waves fetch what follows
+    backward_w(last, bn);
+    const int out = last & 1;
+    if (w == 0) {
+        f32x4_t acc[2];
+        product(out, a.kp[last] >> 5, bw, acc);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            uint16_t h[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = i * 16 + rq + r;
+                const bool on = m0 + row < a.B;
+                const float er = on ? target_error(acc[i][r] + bias, a.Y[src[row]], a.ym, a.yis) : 0.f;
+                const float d = on ? 2.f * er / (float)a.B : 0.f;
+                if ((l & 15) == 0) DZ[(size_t)row * a.zcols + a.zcol[last]] = d;
+                h[r] = f2bf(d);
+                H[out ^ 1][row][l & 15] = (l & 15) == 0 ? h[r] : (uint16_t)0;
+                H[out ^ 1][row][16 + (l & 15)] = 0;
+                if (on && (l & 15) == 0) a.sq[e * a.sqn + m0 + row] = er * er;
+            }
+            if ((l & 15) == 0) *reinterpret_cast<uint64_t *>(DZT + a.zt0[last] * ts + frag_at(0, i * 16 + rq, 1)) = pack4(h);
+        }
+    }
+    __syncthreads();
+    for (int L = last; L > 0; --L) {
+        const int from = (L & 1) ^ 1;
+#pragma unroll
+        for (int kb = 0; kb < IMAXW / 32; ++kb) bw[kb] = bn[kb];
+        if (L > 1) backward_w(L - 1, bn);
+        if (n0 < a.fin[L]) {
+            f32x4_t zz[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) zz[i] = Z[((L - 1) * IWAVES * 2 + i) * 64];
+            f32x4_t acc[2];
+            product(from, (a.fout[L] + 31) >> 5, bw, acc);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                float dz[4];
+                uint16_t h[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = i * 16 + rq + r;
+                    dz[r] = m0 + row < a.B ? silu_back(acc[i][r], zz[i][r]) : 0.f;
+                    DZ[(size_t)row * a.zcols + a.zcol[L - 1] + c] = dz[r];
+                }
+                f2bf4(dz, h);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) H[from ^ 1][i * 16 + rq + r][c] = h[r];
+                *reinterpret_cast<uint64_t *>(DZT + (a.zt0[L - 1] + w) * ts + frag_at(l & 15, i * 16 + rq, 1)) = pack4(h);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Latency-bound as well (the same shape: 31 us, 41 with X and dZ in rows of the
+// batch, of which a load takes 16 half lines): a wave holds a 32 x 32 quarter of its tile and walks
+// the batch in blocks of 32, TKU blocks' operands in flight; a column sum is a
+// chain of B dependent additions per lane with as many rows in flight.
+constexpr int TKU = 4, TSR = 32;
+static_assert(IMR == 32 && IMR % TSR == 0, "a row tile is one block of a weight gradient's k");
+__global__ __launch_bounds__(256) void k_train_weights(const TrainArgs a) {
+    const int ue = a.nsum + a.tile0[a.nl], unit = chiplet_unit(ue * a.mg);
+    if (unit < 0) return;
+    const int e = unit / ue, ub = unit - e * ue;
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
+    const float c1 = a.c1[e], c2 = a.c2[e];
+    float *const p = a.p[e], *const am = a.am[e], *const av = a.av[e];
+    uint16_t *const wt = a.wt[e];
+    if (ub < a.nsum) {
+        const int col = ub * 256 + t;
+        if (col >= a.zcols) return;
+        const float *x = a.DZ + (size_t)e * a.tiles * IMR * a.zcols + col;
+        float s = 0.f, cur[TSR], nxt[TSR];
+#pragma unroll
+        for (int q = 0; q < TSR; ++q) cur[q] = x[(size_t)q * a.zcols];
+        const int nr = a.tiles * IMR;  // rows past the batch hold zeros
+        for (int r0 = 0; r0 < nr; r0 += TSR) {
+            const int r1 = r0 + TSR < nr ? r0 + TSR : r0;
+#pragma unroll
+            for (int q = 0; q < TSR; ++q) nxt[q] = x[(size_t)(r1 + q) * a.zcols];
+#pragma unroll
+            for (int q = 0; q < TSR; ++q) s += cur[q];
+#pragma unroll
+            for (int q = 0; q < TSR; ++q) cur[q] = nxt[q];
+        }
+        int L = 0;
+        while (L + 1 < a.nl && col >= a.zcol[L + 1]) ++L;
+        const int q = a.boff[L] + (col - a.zcol[L]);
+        float v1 = p[q], v2 = am[q], v3 = av[q];
+        adam_update(v1, v2, v3, s, a.adam, c1, c2);
+        p[q] = v1;
+        am[q] = v2;
+        av[q] = v3;
+        return;
+    }
+    const int id = ub - a.nsum;
+    int L = 0;
+    while (L + 1 < a.nl && id >= a.tile0[L + 1]) ++L;
+    const int M = a.fin[L], N = a.fout[L], nt = (N + 63) / 64, k = id - a.tile0[L];
+    const int mt = k / nt * 64 + (w >> 1) * 32, nt0 = k % nt * 64 + (w & 1) * 32;
+    if (mt >= M || nt0 >= N) return;
+    const int nb = a.tiles;
+    const uint16_t *xa[2], *zb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        xa[i] = a.XT + ((size_t)e * a.xtiles + a.xt0[L] + min(mt / 16 + i, (M - 1) / 16)) * nb * 512 + l * 8;
+        zb[i] = a.DZT + ((size_t)e * a.ztiles + a.zt0[L] + min(nt0 / 16 + i, (N - 1) / 16)) * nb * 512 + l * 8;
+    }
+    f32x4_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int b0, bf16x8_t(&A)[TKU][2], bf16x8_t(&B)[TKU][2]) {
+#pragma unroll
+        for (int u = 0; u < TKU; ++u) {
+            const int b = 512 * min(b0 + u, nb - 1);  // past the end: loaded again, not used
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                A[u][i] = *reinterpret_cast<const bf16x8_t *>(xa[i] + b);
+                B[u][i] = *reinterpret_cast<const bf16x8_t *>(zb[i] + b);
+            }
+        }
+    };
+    bf16x8_t A[TKU][2], B[TKU][2], An[TKU][2], Bn[TKU][2];
+    load(0, A, B);
+    for (int b0 = 0; b0 < nb; b0 += TKU) {
+        load(b0 + TKU, An, Bn);
+#pragma unroll
+        for (int u = 0; u < TKU; ++u) {
+            if (b0 + u >= nb) break;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[u][i], B[u][j], acc[i][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < TKU; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                A[u][i] = An[u][i];
+                B[u][i] = Bn[u][i];
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int m = mt + i * 16 + (l >> 4) * 4, n = nt0 + j * 16 + (l & 15);
+            if (m >= M || n >= N) continue;
+            const int q = a.woff[L] + m * N + n;
+            float v1[4], v2[4], v3[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int o = q + (m + r < M ? r * N : 0);
+                v1[r] = p[o];
+                v2[r] = am[o];
+                v3[r] = av[o];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) adam_update(v1[r], v2[r], v3[r], acc[i][j][r], a.adam, c1, c2);
+            uint16_t h[4];
+            f2bf4(v1, h);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (m + r < M) {
+                    p[q + r * N] = v1[r];
+                    am[q + r * N] = v2[r];
+                    av[q + r * N] = v3[r];
+                    if (L) wt[a.wtoff[2 * L + 1] + frag_at(m + r, n, (N + 31) >> 5)] = h[r];
+                } else {
+                    h[r] = 0;
+                }
+            *reinterpret_cast<uint64_t *>(wt + a.wtoff[2 * L] + frag_at(n, m, a.kp[L] >> 5)) = pack4(h);
+        }
 }
 
 __global__ void k_to_bf16(const float *__restrict__ in, uint16_t *__restrict__ out, size_t n) {
@@ -327,6 +742,7 @@ struct CasimMLP {
     size_t wt_per = 0;
     uint64_t pver = 1, wt_ver = 0;
     bool fused_ok() const;
+    size_t wt_offsets(int *off) const;
     void refresh_wt();
     void infer(const float *x, int B, float *out, int ostride);
     // batch workspace
@@ -336,6 +752,18 @@ struct CasimMLP {
     float *dH = nullptr, *dZ = nullptr, *tgt = nullptr, *sq = nullptr;
     uint16_t *dZb = nullptr;
     int *idx = nullptr;
+    // workspace of the two-launch training step (TrainArgs), for tr_members
+    // members and tr_rows batch rows at a time
+    int tr_members = 0, tr_rows = 0;
+    int64_t tr_perm = 0;
+    uint16_t *tr_x = nullptr, *tr_dzt = nullptr;
+    float *tr_dz = nullptr, *tr_z = nullptr, *tr_sq = nullptr;
+    int *tr_idx = nullptr;
+    bool train_fused(int B) const;
+    int train_members(int B) const;
+    void train_reserve(int mg, int B);
+    void train_free();
+    void train_group(int e0, int mg, int epochs, int B, float lr, uint64_t seed, float *loss_out);
 
     void use() { HIPCK(hipSetDevice(dev)); }
     void reserve(int b);
@@ -357,26 +785,40 @@ bool CasimMLP::fused_ok() const {
     return fused && members <= IMAXM && depth + 1 <= IMAXL && n_in <= IMAXW && width <= IMAXW && width % 64 == 0;
 }
 
+// Offsets of the operands of layer g / 2 (k_wt) in a member's copy; the bytes
+// of a member's copy.
+size_t CasimMLP::wt_offsets(int *off) const {
+    size_t per = 0;
+    for (int g = 0; g <= 2 * depth + 1; ++g) {
+        const int n = g & 1 ? fin[g / 2] : fout[g / 2], k = g & 1 ? fout[g / 2] : fin[g / 2];
+        off[g] = (int)per;
+        per += (size_t)((n + 15) & ~15) * ((k + 31) & ~31);
+    }
+    return per;
+}
+
 void CasimMLP::refresh_wt() {
     if (wt && wt_ver == pver) return;
-    std::vector<size_t> off;
-    size_t per = 0;
-    for (int l = 0; l <= depth; ++l) {
-        off.push_back(per);
-        per += (size_t)((fout[l] + 15) & ~15) * ((fin[l] + 31) & ~31);
-    }
+    WtArgs a{};
+    const size_t per = wt_offsets(a.off);
     if (!wt) {
         HIPCK(hipMalloc(&wt, sizeof(uint16_t) * per * members));
         wt_per = per;
     }
-    for (int e = 0; e < members; ++e)
-        for (int l = 0; l <= depth; ++l) {
-            const int kp = (fin[l] + 31) & ~31, np = (fout[l] + 15) & ~15;
-            const size_t n = (size_t)np * kp;
-            hipLaunchKernelGGL(k_wt, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, pb[e] + woff[l],
-                               wt + (size_t)e * wt_per + off[l], fin[l], fout[l], kp, np);
-            HIPCK(hipGetLastError());
-        }
+    size_t most = 0;
+    for (int l = 0; l <= depth; ++l) {
+        a.woff[l] = (int)woff[l];
+        a.fin[l] = fin[l];
+        a.fout[l] = fout[l];
+        most = std::max(most, (size_t)((fout[l] + 31) & ~31) * ((fin[l] + 31) & ~31));
+    }
+    for (int e = 0; e < members; ++e) {
+        a.pb[e] = pb[e];
+        a.wt[e] = wt + (size_t)e * wt_per;
+    }
+    hipLaunchKernelGGL(k_wt, dim3((unsigned)((most + 255) / 256), (unsigned)(2 * depth + 2), (unsigned)members), dim3(256), 0,
+                       stream, a);
+    HIPCK(hipGetLastError());
     wt_ver = pver;
 }
 
@@ -384,13 +826,13 @@ void CasimMLP::refresh_wt() {
 void CasimMLP::infer(const float *x, int B, float *out, int ostride) {
     refresh_wt();
     InferArgs a{};
-    size_t off = 0;
+    int off[2 * IMAXL];
+    (void)wt_offsets(off);
     for (int l = 0; l <= depth; ++l) {
-        a.wtoff[l] = (int)off;
+        a.wtoff[l] = off[2 * l];
         a.kp[l] = (fin[l] + 31) & ~31;
         a.fout[l] = fout[l];
         a.boff[l] = (int)boff[l];
-        off += (size_t)((fout[l] + 15) & ~15) * a.kp[l];
     }
     for (int e = 0; e < members; ++e) {
         a.wt[e] = wt + (size_t)e * wt_per;
@@ -400,9 +842,67 @@ void CasimMLP::infer(const float *x, int B, float *out, int ostride) {
     a.n_in = n_in;
     a.mean = mean;
     a.istd = istd;
-    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((B + IMR - 1) / IMR), (unsigned)members), dim3(64 * IWAVES), 0, stream, x,
-                       B, out, ostride, a);
+    const int big = (B + 63) / 64;
+    if ((size_t)big * members >= INFER_BIG)
+        hipLaunchKernelGGL((k_mlp_infer<2, 4>), dim3((unsigned)big, (unsigned)members), dim3(32 * IWAVES), 0, stream, x, B, out,
+                           ostride, a);
+    else
+        hipLaunchKernelGGL((k_mlp_infer<1, 2>), dim3((unsigned)((B + IMR - 1) / IMR), (unsigned)members), dim3(64 * IWAVES), 0,
+                           stream, x, B, out, ostride, a);
     HIPCK(hipGetLastError());
+}
+
+// Batch rows in whole tiles; columns of a member's X and dZ operands in tiles of 16.
+struct TrainSize {
+    size_t bp, x = 0, z = 0, zc = 0;
+    TrainSize(const CasimMLP *m, int B) : bp((size_t)(B + IMR - 1) / IMR * IMR) {
+        for (int l = 0; l <= m->depth; ++l) {
+            x += (m->fin[l] + 15) / 16 * 16;
+            z += (m->fout[l] + 15) / 16 * 16;
+            zc += m->fout[l];
+        }
+    }
+};
+// Bytes of a member's workspace of the two-launch training step.
+static size_t train_bytes(const CasimMLP *m, int B) {
+    const TrainSize t(m, B);
+    return t.bp * (2 * t.x + 2 * t.z + 4 * t.zc + 4 * (size_t)m->depth * IMAXW);
+}
+
+// The two launches take the shapes of k_mlp_infer; batches past 1 GiB of
+// workspace per member go a layer at a time.
+bool CasimMLP::train_fused(int B) const {
+    return fused_ok() && train_bytes(this, B) <= ((size_t)1 << 30);
+}
+
+// Members that step together: all of them while their workspace is within 1 GiB.
+int CasimMLP::train_members(int B) const {
+    return (int)std::min<size_t>(members, std::max<size_t>(1, ((size_t)1 << 30) / train_bytes(this, B)));
+}
+
+void CasimMLP::train_free() {
+    for (void *q : {(void *)tr_x, (void *)tr_dzt, (void *)tr_dz, (void *)tr_z, (void *)tr_sq, (void *)tr_idx})
+        if (q) (void)hipFree(q);
+    tr_x = tr_dzt = nullptr;
+    tr_dz = tr_z = tr_sq = nullptr;
+    tr_idx = nullptr;
+    tr_members = tr_rows = tr_perm = 0;
+}
+
+void CasimMLP::train_reserve(int mg, int B) {
+    if (mg <= tr_members && B <= tr_rows && rows <= tr_perm) return;
+    HIPCK(hipStreamSynchronize(stream));
+    train_free();
+    const TrainSize t(this, B);
+    HIPCK(hipMalloc(&tr_x, sizeof(uint16_t) * mg * t.x * t.bp));
+    HIPCK(hipMalloc(&tr_dzt, sizeof(uint16_t) * mg * t.z * t.bp));
+    HIPCK(hipMalloc(&tr_dz, sizeof(float) * mg * t.zc * t.bp));
+    HIPCK(hipMalloc(&tr_z, sizeof(float) * mg * t.bp * depth * IMAXW));
+    HIPCK(hipMalloc(&tr_sq, sizeof(float) * mg * rows));
+    HIPCK(hipMalloc(&tr_idx, sizeof(int) * mg * rows));
+    tr_members = mg;
+    tr_rows = B;
+    tr_perm = rows;
 }
 
 void CasimMLP::free_batch() {
@@ -465,6 +965,96 @@ void CasimMLP::backward(int e, int B) {
         hipLaunchKernelGGL(k_silu_back, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, dH, Zl[l - 1], dZ,
                            dZb, n);
         HIPCK(hipGetLastError());
+    }
+}
+
+// Epochs of members e0 .. e0 + mg - 1, which step together.  Each keeps its
+// own row order, as if it were trained alone.
+void CasimMLP::train_group(int e0, int mg, int epochs, int B, float lr, uint64_t seed, float *loss_out) {
+    refresh_wt();  // k_train_weights keeps the transposed weights up to date
+    ++pver;
+    TrainArgs a{};
+    (void)wt_offsets(a.wtoff);
+    for (int l = 0; l <= depth; ++l) {
+        a.kp[l] = (fin[l] + 31) & ~31;
+        a.fin[l] = fin[l];
+        a.fout[l] = fout[l];
+        a.woff[l] = (int)woff[l];
+        a.boff[l] = (int)boff[l];
+        a.xt0[l] = a.xtiles;
+        a.zt0[l] = a.ztiles;
+        a.zcol[l] = a.zcols;
+        a.xtiles += (fin[l] + 15) / 16;
+        a.ztiles += (fout[l] + 15) / 16;
+        a.zcols += fout[l];
+        a.tile0[l + 1] = a.tile0[l] + (fin[l] + 63) / 64 * ((fout[l] + 63) / 64);
+    }
+    for (int e = 0; e < mg; ++e) {
+        a.wt[e] = wt + (size_t)(e0 + e) * wt_per;
+        a.p[e] = p[e0 + e];
+        a.am[e] = am[e0 + e];
+        a.av[e] = av[e0 + e];
+    }
+    a.nl = depth + 1;
+    a.mg = mg;
+    a.nsum = (a.zcols + 255) / 256;
+    a.n_in = n_in;
+    a.B = B;
+    a.tiles = (B + IMR - 1) / IMR;
+    a.mean = mean, a.istd = istd, a.X = X, a.Y = Y;
+    a.rows = a.sqn = rows;
+    a.ym = ym;
+    a.yis = 1.f / ys;
+    a.XT = tr_x, a.DZT = tr_dzt, a.DZ = tr_dz, a.Z = tr_z;
+    a.adam = {lr, 0.9f, 0.999f, 1e-8f};
+    std::vector<std::mt19937_64> gen;
+    for (int e = e0; e < e0 + mg; ++e) gen.emplace_back(seed * 1315423911ull + (uint64_t)e * 2654435761ull + 17);
+    std::vector<int> perm((size_t)mg * rows);
+    const int64_t nb = rows / B;
+    struct Event {
+        hipEvent_t e = nullptr;
+        ~Event() {
+            if (e) (void)hipEventDestroy(e);
+        }
+    } copied;
+    HIPCK(hipEventCreateWithFlags(&copied.e, hipEventDisableTiming));
+    for (int ep = 0; ep < epochs; ++ep) {
+        // the last epoch's order has left the host buffer; its batches still run
+        if (ep) HIPCK(hipEventSynchronize(copied.e));
+        for (int e = 0; e < mg; ++e) {
+            int *q = perm.data() + (size_t)e * rows;
+            std::iota(q, q + rows, 0);
+            std::shuffle(q, q + rows, gen[e]);
+        }
+        HIPCK(hipMemcpyAsync(tr_idx, perm.data(), sizeof(int) * perm.size(), hipMemcpyHostToDevice, stream));
+        HIPCK(hipEventRecord(copied.e, stream));
+        for (int64_t b = 0; b < nb; ++b) {
+            a.perm = tr_idx + b * B;
+            a.sq = tr_sq + b * B;
+            for (int e = 0; e < mg; ++e) {
+                const int t = ++steps[e0 + e];
+                a.c1[e] = 1.f - std::pow(a.adam.b1, (float)t);
+                a.c2[e] = 1.f - std::pow(a.adam.b2, (float)t);
+            }
+            hipLaunchKernelGGL(k_train_rows, dim3(chiplet_grid(a.tiles * mg)), dim3(64 * IWAVES), 0, stream, a);
+            HIPCK(hipGetLastError());
+            hipLaunchKernelGGL(k_train_weights, dim3(chiplet_grid((a.nsum + a.tile0[a.nl]) * mg)), dim3(256), 0, stream,
+                               a);
+            HIPCK(hipGetLastError());
+        }
+    }
+    for (int e = e0; e < e0 + mg; ++e) {
+        hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, stream, p[e], pb[e], P);
+        HIPCK(hipGetLastError());
+    }
+    std::vector<float> sq((size_t)mg * rows);
+    HIPCK(hipMemcpyAsync(sq.data(), tr_sq, sizeof(float) * sq.size(), hipMemcpyDeviceToHost, stream));
+    HIPCK(hipStreamSynchronize(stream));
+    wt_ver = pver;
+    for (int e = 0; e < mg && loss_out; ++e) {
+        double sum = 0.0;
+        for (int64_t i = 0; i < nb * B; ++i) sum += sq[(size_t)e * rows + i];
+        loss_out[e0 + e] = (float)(sum / (double)(nb * B));
     }
 }
 
@@ -658,6 +1248,7 @@ int casim_mlp_destroy(CasimMLP *m) {
     (void)hipSetDevice(m->dev);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     m->free_batch();
+    m->train_free();
     for (auto v : {&m->p, &m->g, &m->am, &m->av})
         for (float *q : *v) (void)hipFree(q);
     for (uint16_t *q : m->pb) (void)hipFree(q);
@@ -735,13 +1326,18 @@ int casim_mlp_train(CasimMLP *m, int32_t epochs, int32_t batch, float lr, uint64
         REQUIRE(epochs >= 1 && batch >= 1, CASIM_E_INVALID, "bad epochs/batch");
         m->use();
         const int B = (int)std::min<int64_t>(batch, m->rows);
+        if (m->train_fused(B)) {
+            const int mg = m->train_members(B);
+            m->train_reserve(mg, B);
+            for (int e0 = 0; e0 < m->members; e0 += mg)
+                m->train_group(e0, std::min(mg, m->members - e0), epochs, B, lr, seed, loss_out);
+            return;
+        }
         m->reserve(B);
         std::vector<int> perm(m->rows);
-        const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+        const AdamArgs adam{lr, 0.9f, 0.999f, 1e-8f};
         const float yis = 1.f / m->ys;
-        float *sq_h = nullptr;
         std::vector<float> sq(B);
-        (void)sq_h;
         ++m->pver;  // the transposed inference weights follow the parameters
         for (int e = 0; e < m->members; ++e) {
             std::mt19937_64 gen(seed * 1315423911ull + (uint64_t)e * 2654435761ull + 17);
@@ -766,9 +1362,9 @@ int casim_mlp_train(CasimMLP *m, int32_t epochs, int32_t batch, float lr, uint64
                     HIPCK(hipGetLastError());
                     m->backward(e, B);
                     const int t = ++m->steps[e];
-                    const float c1 = 1.f - std::pow(b1, (float)t), c2 = 1.f - std::pow(b2, (float)t);
+                    const float c1 = 1.f - std::pow(adam.b1, (float)t), c2 = 1.f - std::pow(adam.b2, (float)t);
                     hipLaunchKernelGGL(k_adam, dim3((unsigned)((m->P + 255) / 256)), dim3(256), 0, m->stream, m->p[e],
-                                       m->g[e], m->am[e], m->av[e], m->pb[e], m->P, lr, b1, b2, eps, c1, c2);
+                                       m->g[e], m->am[e], m->av[e], m->pb[e], m->P, adam, c1, c2);
                     HIPCK(hipGetLastError());
                     if (keep) {
                         HIPCK(hipMemcpyAsync(sq.data(), m->sq, sizeof(float) * B, hipMemcpyDeviceToHost, m->stream));

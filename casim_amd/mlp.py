@@ -118,7 +118,7 @@ class MLP:
         return float(loss[0]), g
 
     def set_fused(self, on):
-        """Fused inference kernel (default) or the per-layer GEMMs; same outputs."""
+        """Fused inference and training kernels (default) or the per-layer ones; same outputs."""
         abi.check(self.lib.casim_mlp_set_fused_inference(self.h, int(bool(on))))
 
     def predict(self, x):

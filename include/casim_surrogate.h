@@ -73,8 +73,9 @@ int casim_mlp_predict(CasimMLP *m, const float *x, int64_t rows, float *mean, fl
  * quasi-stationary path run every layer of a member in one fused kernel
  * (activations in LDS, BF16 MFMA, FP32 accumulation) where the shape allows
  * it (members <= 8, layers <= 8, inputs and width <= 256, width a multiple
- * of 64); 0 selects the per-layer GEMM and bias kernels.  The outputs are
- * the same bits either way. */
+ * of 64), and casim_mlp_train takes every member's step in two launches; 0
+ * selects the per-layer GEMM and bias kernels.  The outputs are the same bits
+ * either way. */
 int casim_mlp_set_fused_inference(CasimMLP *m, int32_t on);
 
 /*
