@@ -759,6 +759,10 @@ struct CasimMLP {
     uint16_t *tr_x = nullptr, *tr_dzt = nullptr;
     float *tr_dz = nullptr, *tr_z = nullptr, *tr_sq = nullptr;
     int *tr_idx = nullptr;
+    // features and outputs of casim_mlp_predict, for pr_rows rows at a time
+    int pr_rows = 0;
+    float *pr_x = nullptr, *pr_out = nullptr;
+    void predict_reserve(int b);
     bool train_fused(int B) const;
     int train_members(int B) const;
     void train_reserve(int mg, int B);
@@ -878,6 +882,20 @@ bool CasimMLP::train_fused(int B) const {
 // Members that step together: all of them while their workspace is within 1 GiB.
 int CasimMLP::train_members(int B) const {
     return (int)std::min<size_t>(members, std::max<size_t>(1, ((size_t)1 << 30) / train_bytes(this, B)));
+}
+
+// Rows of a chunk of casim_mlp_predict, which bounds what a handle keeps for it.
+constexpr int PREDICT_ROWS = 65536;
+
+void CasimMLP::predict_reserve(int b) {
+    if (b <= pr_rows) return;
+    if (pr_x) (void)hipFree(pr_x);
+    if (pr_out) (void)hipFree(pr_out);
+    pr_x = pr_out = nullptr;
+    pr_rows = 0;
+    HIPCK(hipMalloc(&pr_x, sizeof(float) * (size_t)b * n_in));
+    HIPCK(hipMalloc(&pr_out, sizeof(float) * (size_t)b * (members + 2)));
+    pr_rows = b;
 }
 
 void CasimMLP::train_free() {
@@ -1149,16 +1167,18 @@ __global__ void k_na_collect(const float *__restrict__ z, float *__restrict__ ou
     if (r < rows) out[r] = z[r];
 }
 
-// Mean and relative spread of exp(y * ys + ym) over the members, in the
-// arithmetic of casim_mlp_predict's host reduction.
-__global__ void k_na_reduce(const float *__restrict__ out, int members, int cap, int rows, float ys, float ym,
-                            float *__restrict__ mean, float *__restrict__ spread) {
+// Mean and relative spread of exp(y * ys + ym) over the members; with keep, out
+// becomes y * ys + ym.  A few us for 55003 rows of five members, where the same
+// sums on the host, member by member after a copy of its outputs, took 1 ms.
+__global__ void k_na_reduce(float *__restrict__ out, int members, int cap, int rows, float ys, float ym,
+                            float *__restrict__ mean, float *__restrict__ spread, int keep) {
 #pragma clang fp contract(off)
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     double s = 0, s2 = 0;
     for (int e = 0; e < members; ++e) {
         const float o = out[(size_t)e * cap + r] * ys + ym;
+        if (keep) out[(size_t)e * cap + r] = o;
         const double v = exp((double)o);
         s += v;
         s2 += v * v;
@@ -1253,7 +1273,7 @@ int casim_mlp_destroy(CasimMLP *m) {
         for (float *q : *v) (void)hipFree(q);
     for (uint16_t *q : m->pb) (void)hipFree(q);
     if (m->wt) (void)hipFree(m->wt);
-    for (void *q : {(void *)m->mean, (void *)m->istd, (void *)m->X, (void *)m->Y, (void *)m->perm_d})
+    for (void *q : {(void *)m->mean, (void *)m->istd, (void *)m->X, (void *)m->Y, (void *)m->perm_d, (void *)m->pr_x, (void *)m->pr_out})
         if (q) (void)hipFree(q);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
@@ -1419,56 +1439,40 @@ int casim_mlp_predict(CasimMLP *m, const float *x, int64_t rows, float *mean, fl
     return guard([&] {
         REQUIRE(m && x && rows >= 1, CASIM_E_INVALID, "bad arguments");
         m->use();
-        const int chunk = (int)std::min<int64_t>(rows, 65536);
+        const int chunk = (int)std::min<int64_t>(rows, PREDICT_ROWS);
         const bool fused = m->fused_ok();
         if (!fused) m->reserve(chunk);
-        float *dx = nullptr, *dout = nullptr;
-        HIPCK(hipMalloc(&dx, sizeof(float) * (size_t)chunk * m->n_in));
-        if (fused) HIPCK(hipMalloc(&dout, sizeof(float) * (size_t)chunk * m->members));
-        std::vector<float> out((size_t)m->members * rows);
-        std::vector<float> tmp(chunk);
+        m->predict_reserve(chunk);
+        const int B0 = m->pr_rows;  // row stride of the device outputs
+        float *const raw = m->pr_out, *const mu = raw + (size_t)m->members * B0, *const sd = mu + B0;
         for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
             const int B = (int)std::min<int64_t>(chunk, rows - r0);
-            HIPCK(hipMemcpyAsync(dx, x + r0 * m->n_in, sizeof(float) * (size_t)B * m->n_in, hipMemcpyHostToDevice,
+            HIPCK(hipMemcpyAsync(m->pr_x, x + r0 * m->n_in, sizeof(float) * (size_t)B * m->n_in, hipMemcpyHostToDevice,
                                  m->stream));
             if (fused) {
-                m->infer(dx, B, dout, B);
+                m->infer(m->pr_x, B, raw, B0);
+            } else {
+                const size_t n = (size_t)B * m->n_in;
+                hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, m->pr_x,
+                                   (const float *)nullptr, (const int *)nullptr, B, m->n_in, m->mean, m->istd, 0.f, 1.f,
+                                   m->Xl[0], (float *)nullptr);
+                HIPCK(hipGetLastError());
                 for (int e = 0; e < m->members; ++e) {
-                    HIPCK(hipMemcpyAsync(tmp.data(), dout + (size_t)e * B, sizeof(float) * B, hipMemcpyDeviceToHost,
+                    m->forward(e, B);
+                    HIPCK(hipMemcpyAsync(raw + (size_t)e * B0, m->Zl[m->depth], sizeof(float) * B, hipMemcpyDeviceToDevice,
                                          m->stream));
-                    HIPCK(hipStreamSynchronize(m->stream));
-                    for (int i = 0; i < B; ++i) out[(size_t)e * rows + r0 + i] = tmp[i] * m->ys + m->ym;
                 }
-                continue;
             }
-            const size_t n = (size_t)B * m->n_in;
-            hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, dx,
-                               (const float *)nullptr, (const int *)nullptr, B, m->n_in, m->mean, m->istd, 0.f, 1.f,
-                               m->Xl[0], (float *)nullptr);
+            hipLaunchKernelGGL(casim::k_na_reduce, dim3((B + 255) / 256), dim3(256), 0, m->stream, raw, m->members, B0, B,
+                               m->ys, m->ym, mu, sd, 1);
             HIPCK(hipGetLastError());
-            for (int e = 0; e < m->members; ++e) {
-                m->forward(e, B);
-                HIPCK(hipMemcpyAsync(tmp.data(), m->Zl[m->depth], sizeof(float) * B, hipMemcpyDeviceToHost,
-                                     m->stream));
-                HIPCK(hipStreamSynchronize(m->stream));
-                for (int i = 0; i < B; ++i) out[(size_t)e * rows + r0 + i] = tmp[i] * m->ys + m->ym;
-            }
+            if (mean) HIPCK(hipMemcpyAsync(mean + r0, mu, sizeof(float) * B, hipMemcpyDeviceToHost, m->stream));
+            if (spread) HIPCK(hipMemcpyAsync(spread + r0, sd, sizeof(float) * B, hipMemcpyDeviceToHost, m->stream));
+            if (member_out)
+                HIPCK(hipMemcpy2DAsync(member_out + r0, sizeof(float) * rows, raw, sizeof(float) * B0, sizeof(float) * B,
+                                       m->members, hipMemcpyDeviceToHost, m->stream));
         }
-        (void)hipFree(dx);
-        if (dout) (void)hipFree(dout);
-        for (int64_t i = 0; i < rows; ++i) {
-            double s = 0, s2 = 0;
-            for (int e = 0; e < m->members; ++e) {
-                const double v = std::exp((double)out[(size_t)e * rows + i]);
-                s += v;
-                s2 += v * v;
-            }
-            const double mu = s / m->members;
-            const double var = std::max(0.0, s2 / m->members - mu * mu);
-            if (mean) mean[i] = (float)mu;
-            if (spread) spread[i] = (float)(mu > 0 ? std::sqrt(var) / mu : 0.0);
-        }
-        if (member_out) std::memcpy(member_out, out.data(), sizeof(float) * out.size());
+        HIPCK(hipStreamSynchronize(m->stream));
     });
 }
 
@@ -1525,8 +1529,8 @@ int casim_mlp_predict_noalloc(CasimMLP *m, const float *x, int64_t rows, float *
                                outm + (size_t)e * cap, B);
             HIPCK(hipGetLastError());
         }
-        hipLaunchKernelGGL(casim::k_na_reduce, dim3((B + 255) / 256), dim3(256), 0, st, (const float *)outm, m->members,
-                           cap, B, m->ys, m->ym, mean, spread);
+        hipLaunchKernelGGL(casim::k_na_reduce, dim3((B + 255) / 256), dim3(256), 0, st, outm, m->members, cap, B, m->ys, m->ym,
+                           mean, spread, 0);
         HIPCK(hipGetLastError());
     });
 }
