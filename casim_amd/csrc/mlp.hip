@@ -125,6 +125,23 @@ __global__ __launch_bounds__(256) void k_gemm(const uint16_t *__restrict__ A, in
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.f / (1.f + __expf(-z)); }
 
+// sigmoidf_ of four values.  1 / d for 1 <= d <= 2^125 by the hardware's
+// reciprocal and one Newton step, which gives the correctly rounded quotient,
+// the compiler's result, for every float in that range (compared one by one);
+// its general division takes 11 operations.  Below -86 the general one.
+__device__ __forceinline__ void sigmoid4(const float (&z)[4], float (&s)[4]) {
+    if (fminf(fminf(z[0], z[1]), fminf(z[2], z[3])) < -86.f) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = sigmoidf_(z[i]);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float d = 1.f + __expf(-z[i]), y = __builtin_amdgcn_rcpf(d);
+        s[i] = __builtin_fmaf(__builtin_fmaf(-d, y, 1.f), y, y);
+    }
+}
+
 // f2bf of four values by the conversion instruction (two values each, the same
 // rounding)
 __device__ __forceinline__ void f2bf4(const float (&f)[4], uint16_t (&h)[4]) {
@@ -158,7 +175,8 @@ __global__ void k_bias_act(float *__restrict__ Z, const float *__restrict__ b, u
 // their way while a layer runs.  Many rows: eight waves with 32 columns each, 64
 // rows, two workgroups per CU.  The weights are then read half as often and the
 // rows' operands from LDS feed two products; what bounds it is the SiLU, about
-// 25 vector operations per activation.  Times in us for five members of width
+// 14 vector operations per activation (55003 rows: 249 us, 276 with the
+// compiler's division in it, 25 operations).  Times in us for five members of width
 // 256, depth 4 (before: weights in plain rows, 32 rows per workgroup):
 //   rows        512   2048   4096   8192   16384   55003
 //   before       -      -      -      -      195     658
@@ -286,9 +304,11 @@ __global__ __launch_bounds__(64 * IWAVES / CT, 4) void k_mlp_infer(const float *
                         for (int r = 0; r < 4; ++r)
                             if (m0 + row + r < rows) out[(size_t)e * ostride + m0 + row + r] = z[r];
                     } else {
+                        float sg[4];
                         uint16_t h[4];
+                        sigmoid4(z, sg);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) z[r] *= sigmoidf_(z[r]);
+                        for (int r = 0; r < 4; ++r) z[r] *= sg[r];
                         f2bf4(z, h);
 #pragma unroll
                         for (int r = 0; r < 4; ++r) H[src ^ 1][row + r][col] = h[r];
@@ -305,18 +325,15 @@ __global__ __launch_bounds__(64 * IWAVES / CT, 4) void k_mlp_infer(const float *
     }
 }
 
-// dH * SiLU'(z)
-__device__ __forceinline__ float silu_back(float dH, float z) {
-    const float s = sigmoidf_(z);
-    return dH * s * (1.f + z * (1.f - s));
-}
+// dH * SiLU'(z), s the sigmoid of z
+__device__ __forceinline__ float silu_back(float dH, float z, float s) { return dH * s * (1.f + z * (1.f - s)); }
 
 // dZ = dH * SiLU'(Z), kept in FP32 (bias gradient) and BF16 (GEMM operand).
 __global__ void k_silu_back(const float *__restrict__ dH, const float *__restrict__ Z, float *__restrict__ dZ,
                             uint16_t *__restrict__ dZb, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float d = silu_back(dH[i], Z[i]);
+    const float d = silu_back(dH[i], Z[i], sigmoidf_(Z[i]));
     dZ[i] = d;
     dZb[i] = f2bf(d);
 }
@@ -509,14 +526,13 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 f32x4_t zz;
-                float f[4];
+                float z[4], f[4];
                 uint16_t h[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float z = acc[i][r] + bias;
-                    zz[r] = z;
-                    f[r] = z * sigmoidf_(z);
-                }
+                for (int r = 0; r < 4; ++r) zz[r] = z[r] = acc[i][r] + bias;
+                sigmoid4(z, f);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) f[r] *= z[r];
                 f2bf4(f, h);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
@@ -571,12 +587,14 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
             product(from, (a.fout[L] + 31) >> 5, bw, acc);
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                float dz[4];
+                const float z[4] = {zz[i][0], zz[i][1], zz[i][2], zz[i][3]};
+                float dz[4], sg[4];
                 uint16_t h[4];
+                sigmoid4(z, sg);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = i * 16 + rq + r;
-                    dz[r] = m0 + row < a.B ? silu_back(acc[i][r], zz[i][r]) : 0.f;
+                    dz[r] = m0 + row < a.B ? silu_back(acc[i][r], z[r], sg[r]) : 0.f;
                     DZ[(size_t)row * a.zcols + a.zcol[L - 1] + c] = dz[r];
                 }
                 f2bf4(dz, h);

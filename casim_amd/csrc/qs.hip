@@ -249,18 +249,25 @@ __global__ __launch_bounds__(64 * QS_FWAVES) void k_qs_features(QsDev q) {
 
 // SRPool::Run (SRPool.cpp:70-89) over an interval dt with a fixed open set:
 // I(c) = c * geff (mouth [Ca2+] proportional to c within the interval),
-// explicit steps of at most 1 us, operations in the pool's order.
+// explicit steps of at most 1 us: c += h / beta (Iref - I), beta = 1 + nK cq /
+// kc^2 with kc = kcq + c.  A step depends on the last one, so its latency is
+// all that counts: h / beta = h kc^2 / (kc^2 + nK cq) leaves one reciprocal (to
+// full precision by two Newton steps, the second folded into the update), where
+// the pool's form divides three times, two of them in a chain.
+// 300 sites over 5 ms: k_qs_event 637 us per round before, 283 with this form,
+// 220 with the step to t_max beside it on a second lane.
 __device__ double jsr_advance(const QsDev &q, double c, double geff, double dt) {
-#pragma clang fp contract(off)
     double n = ceil(dt / 1e-3);
     if (n < 1.0) n = 1.0;
     if (n > 1e6) n = 1e6;
-    const double h = dt / n;
-    for (double k = 0; k < n; k += 1.0) {
-        const double kc = q.kcq + c;
-        const double beta = 1 + q.ncq * q.kcq * q.cq / (kc * kc);
-        const double Iref = (q.nsr - c) / q.tau;
-        c = c + h / beta * (Iref - c * geff * q.Vr);
+    const double h = dt / n, A = q.ncq * q.kcq * q.cq, f0 = h * (q.nsr / q.tau), f1 = h * (1.0 / q.tau + geff * q.Vr);
+    for (int k = (int)n; k > 0; --k) {
+        const double kc = q.kcq + c, k2 = kc * kc, d = __builtin_fma(kc, kc, A);
+        const double g = k2 * __builtin_fma(-f1, c, f0);
+        const double y0 = __builtin_amdgcn_rcp(d);
+        const double y = __builtin_fma(__builtin_fma(-d, y0, 1.0), y0, y0);
+        const double e = __builtin_fma(-d, y, 1.0), u = g * y;  // g / d = u (1 + e)
+        c = __builtin_fma(u, e, c + u);
     }
     return c;
 }
@@ -383,26 +390,33 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
         if (b0) idx = __ffsll((long long)b0) - 1;
         else if (b1) idx = 64 + __ffsll((long long)b1) - 1;
     }
-    if (lane != 0) return;
-    const double dtw = -log(u1) * (1.0 / total);
-    const double t = q.t[s] + dtw;
-    (void)mrg::draw(S6);  // MakeTransition(runif())
+    double dtw = 0.0, cw = 0.0;
+    if (lane == 0) dtw = -log(u1) * (1.0 / total);
     if (q.deplete) {
-        // the jSR over the interval before the event, with this interval's open set
-        const double c0 = q.jsr[s];
+        // the jSR over the interval before the event, with this interval's open
+        // set: every channel's share of the conductance on its lane, summed in
+        // channel order
+        const double c0 = q.jsr[s], tmax = q.t_max - q.t[s];
+        for (int i = lane; i < n; i += 64) pcv[i] = q.state[off + i] == 1 ? q.gch * (1.0 - (double)cav[i] / c0) : 0.0;
+        __syncthreads();
+        dtw = __shfl(dtw, 0);
+        if (lane > 1) return;
         double geff = 0.0;
-        for (int i = 0; i < n; ++i)
-            if (q.state[off + i] == 1) geff += q.gch * (1.0 - (double)cav[i] / c0);
-        const double c1 = jsr_advance(q, c0, geff, dtw);
-        q.jsr[s] = c1;
-        // lowest jSR over [0, t_max], what a run of that length observes
-        if (t <= q.t_max) {
-            if (c1 < q.jsr_min[s]) q.jsr_min[s] = c1;
-        } else if (q.t[s] < q.t_max) {
-            const double cw = jsr_advance(q, c0, geff, q.t_max - q.t[s]);
-            if (cw < q.jsr_min[s]) q.jsr_min[s] = cw;
+        for (int i = 0; i < n; ++i) geff += pcv[i];
+        // lane 1 meanwhile goes to t_max where the event lies past it: the lowest
+        // jSR over [0, t_max] is what a run of that length observes
+        const bool past = q.t[s] + dtw > q.t_max;
+        cw = lane == 0 || (past && tmax > 0.0) ? jsr_advance(q, c0, geff, lane == 0 ? dtw : tmax) : INFINITY;
+        const double c1 = cw, c2 = __shfl(cw, 1);
+        if (lane == 0) {
+            q.jsr[s] = c1;
+            const double low = past ? c2 : c1;
+            if (low < q.jsr_min[s]) q.jsr_min[s] = low;
         }
     }
+    if (lane != 0) return;
+    const double t = q.t[s] + dtw;
+    (void)mrg::draw(S6);  // MakeTransition(runif())
     if (q.trace) {
         // IndChannelCREAnalyzer.cpp:78-84: bins up to the next record's time
         // take the current count
