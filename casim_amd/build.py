@@ -30,7 +30,7 @@ UNITS = [
     ("mlp.hip", []),
     ("qs.hip", []),
     ("cytosol_box.hip", []),
-    ("resident.hip", []),
+    ("resident.hip", []), ("resident2d.hip", []),
     ("sweep_inst.hip", ["-DCASIM_SWEEP_FP64=1", "-DCASIM_SWEEP_DIM=3"]),
     ("sweep_inst.hip", ["-DCASIM_SWEEP_FP64=1", "-DCASIM_SWEEP_DIM=2"]),
     ("sweep_inst.hip", ["-DCASIM_SWEEP_FP64=0", "-DCASIM_SWEEP_DIM=3"]),

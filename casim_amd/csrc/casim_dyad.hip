@@ -548,6 +548,7 @@ int casim_dyad_destroy(CasimDyad *d) {
     d->clear_graphs();
     casim::box_free(d);
     casim::resident_free(d);
+    casim::site2d_free(d);
     void *ptrs[] = {d->g[0], d->g[1], d->f[0], d->f[1], d->d_off, d->d_node, d->d_type, d->d_perm, d->d_snode,
                     d->d_sperm, d->d_state, d->d_chans, d->d_rng, d->d_rng0, d->d_jump, d->d_mouths, d->d_jsr, d->d_sJ,
                     d->d_snap, d->d_pg, d->d_pjv, d->d_totals, d->d_rim_ions, d->d_rim_bound, d->d_eff, d->d_stats, d->Ch.trace};
@@ -832,14 +833,17 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
         REQUIRE(!d->box || k_steps % M == 0, CASIM_E_INVALID,
                 "with a cytosol box, k_steps must be a multiple of its substeps");
         d->use();
-        if (casim::resident_ok(d, k_steps)) {
+        const bool flat = casim::site2d_ok(d);
+        if (flat || casim::resident_ok(d, k_steps)) {
             for (int32_t left = k_steps; left > 0;) {
                 const int32_t kc = std::min(left, (int32_t)2048);
                 left -= kc;
-                casim::resident_steps(d, dt, kc);
+                flat ? casim::site2d_steps(d, dt, kc) : casim::resident_steps(d, dt, kc);
+                // the update that the next launch's first step expects
+                if (d->Q.on && d->Q.cyto) d->launch_rim(d->Q.cions, d->Q.cbb);
+                d->launch_efflux();
+                d->launch_channels(CH_SNAPSHOT | CH_CURRENTS | CH_ACCUMULATE | CH_POOL_UPDATE, dt);
             }
-            d->launch_efflux();
-            d->launch_channels(CH_SNAPSHOT | CH_CURRENTS | CH_ACCUMULATE | CH_POOL_UPDATE, dt);
             return;
         }
         // One captured graph covers at most 2048 steps, a whole number of

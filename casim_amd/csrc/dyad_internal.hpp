@@ -58,6 +58,7 @@ std::vector<double> buffer_equilibrium(const std::vector<double> &kon, const std
                                        const std::vector<double> &c, double total);
 struct CytoBox;  // 3D cytosol box around each site (cytosol_box.hip)
 struct Resident;  // plan and exchange buffers of the steps with the state on the chip (resident.hip)
+struct Site2D;    // tables of the 2D steps with the state on the chip (resident2d.hip)
 }  // namespace casim
 
 struct CasimDyad {
@@ -95,6 +96,7 @@ struct CasimDyad {
     casim::CytoBox *box = nullptr;  // cytosol box (null when not attached)
     casim::Resident *res = nullptr;  // made by the first step that it can take
     bool res_tried = false;
+    casim::Site2D *s2d = nullptr;
     // the sites and stream the pair and channel launchers work on (all sites
     // on `stream` unless casim_dyad_step splits the batch)
     int range_s0 = 0, range_n = -1;
@@ -149,6 +151,10 @@ bool resident_ok(CasimDyad *d, int k_steps);
 void resident_steps(CasimDyad *d, double dt, int k);
 void resident_check(const CasimDyad *d);
 void resident_free(CasimDyad *d);
+// The same for 2D sites that fit one CU (resident2d.hip).
+bool site2d_ok(const CasimDyad *d);
+void site2d_steps(CasimDyad *d, double dt, int k);
+void site2d_free(CasimDyad *d);
 int layout_id(const Params &p);  // compile-time species layout that fits, or 0 (casim_dyad.hip)
 }  // namespace casim
 
