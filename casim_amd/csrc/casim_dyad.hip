@@ -64,6 +64,11 @@ std::vector<double> buffer_equilibrium(const std::vector<double> &kon, const std
 
 // The compile-time species layout (Layout<LY>) matching the run-time one, or 0.
 int layout_id(const Params &p) {
+    if (p.ni == 2 && p.nb == 4 && p.nu == 3 && p.n_grid == 6 && p.n_face == 0) {
+        for (int b = 0; b < 4; ++b)
+            if (p.bion[b] != Layout<3>::bion[b] || p.bbuf[b] != Layout<3>::bbuf[b]) return 0;
+        return 3;
+    }
     if (p.ni != 1 || p.nb != 3 || p.nu != 3 || p.sl[0] || p.Db[0] == 0.0 || p.Db[1] == 0.0 || p.Db[2] != 0.0)
         return 0;
     for (int ly = 1; ly <= 2; ++ly) {

@@ -398,6 +398,8 @@ __device__ __forceinline__ void st_off(T *base, unsigned boff, T v) {
 // buffer and diffusing A and B.  LY = 0 reads all of it from Params.
 //  1: one ion; buffers A, B mobile, F on the z-faces (Ca-A, Ca-B, Ca-F)
 //  2: one ion; buffers A, B mobile, F fixed on every node
+//  3: two ions; buffer A binds both, B and C the first one, none on the z-faces
+//     (which diffuse and which ion has a sarcolemmal buffer comes from Params)
 template <int LY>
 struct Layout {
     static constexpr bool fixed = false;
@@ -418,6 +420,13 @@ struct Layout<2> {
     static constexpr int bion[3] = {0, 0, 0}, bbuf[3] = {0, 1, 2}, bface[3] = {0, 0, 0}, bslot[3] = {1, 2, 3};
     static constexpr int ufaces[3] = {0, 0, 0};
 };
+template <>
+struct Layout<3> {
+    static constexpr bool fixed = true;
+    static constexpr int nu = 3;
+    static constexpr int bion[4] = {0, 0, 0, 1}, bbuf[4] = {0, 1, 2, 0}, bface[4] = {0, 0, 0, 0}, bslot[4] = {2, 3, 4, 5};
+    static constexpr int ufaces[3] = {0, 0, 0};
+};
 template <int LY> __device__ __forceinline__ int ly_bion(const Params &p, int b) {
     if constexpr (Layout<LY>::fixed) return Layout<LY>::bion[b]; else return p.bion[b];
 }
@@ -432,11 +441,11 @@ template <int LY> __device__ __forceinline__ int ly_bslot(const Params &p, int b
 }
 // sarcolemmal buffer of ion j present (Params::sl)
 template <int LY> __device__ __forceinline__ bool ly_sl(const Params &p, int j) {
-    if constexpr (Layout<LY>::fixed) return false; else return p.sl[j] != 0;
+    if constexpr (Layout<LY>::fixed && LY != 3) return false; else return p.sl[j] != 0;
 }
 // bound field b diffuses (a grid field with D != 0)
 template <int LY> __device__ __forceinline__ bool ly_mobile(const Params &p, int b) {
-    if constexpr (Layout<LY>::fixed) return !Layout<LY>::bface[b] && b < 2; else return p.Db[b] != 0.0;
+    if constexpr (Layout<LY>::fixed && LY != 3) return !Layout<LY>::bface[b] && b < 2; else return p.Db[b] != 0.0;
 }
 template <int LY> __device__ __forceinline__ double ly_total(const Params &p, int u, int z) {
     int faces;

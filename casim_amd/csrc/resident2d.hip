@@ -67,7 +67,8 @@ struct PlaneNbr {
 // (node_update), k_channels, k_efflux, pool_update_site, pool_advance_site and
 // k_rim in their order, so the values are the same bits.
 // What bounds it: the slowest of the three roles between the barriers (100 sites
-// of 31 x 41 nodes with two ions and every compartment: 9.1 us per step; four
+// of 31 x 41 nodes with two ions and every compartment: 7.0 us per step, 9.1
+// with the species layout read at run time, 6.6 without the grid update; four
 // launches of 107 us together before).  A site's state does not leave the CU
 // and there is no launch per step, so any number of steps and sites gains.
 template <typename T, int NI, int NB, int LY, int NT>
@@ -665,7 +666,9 @@ void site2d_steps(CasimDyad *d, double dt, int k) {
     a.cb = d->s2d->cb, a.ci = d->s2d->ci, a.ctot = d->s2d->ctot;
     const size_t lds = lds_bytes(d);
     const bool f64 = d->precision == CASIM_FP64;
-    if (p.ni == 1) {
+    if (layout_id(p) == 3) {
+        f64 ? launch<double, 2, 4, 3>(d, dt, a, lds) : launch<float, 2, 4, 3>(d, dt, a, lds);
+    } else if (p.ni == 1) {
         f64 ? launch<double, 1, 3, 2>(d, dt, a, lds) : launch<float, 1, 3, 2>(d, dt, a, lds);
     } else {
         f64 ? launch<double, 2, 4, 0>(d, dt, a, lds) : launch<float, 2, 4, 0>(d, dt, a, lds);

@@ -77,6 +77,7 @@ void sweep2_species(CasimDyad *d, double dt) {
     const int ly = layout_id(p);
     if (DIM == 3 && ly == 1) return sweep2_slots<T, DIM, 1, 3, 3, 1, 1>(d, dt);
     if (ly == 2) return sweep2_slots<T, DIM, 1, 3, 4, 0, 2>(d, dt);
+    if (ly == 3) return sweep2_slots<T, DIM, 2, 4, 6, 0, 3>(d, dt);
     if (p.ni == 2 && p.nb == 4 && p.n_grid == 6 && p.n_face == 0) return sweep2_slots<T, DIM, 2, 4, 6, 0, 0>(d, dt);
     return sweep2_slots<T, DIM, 0, 0, 0, 0, 0>(d, dt);
 }
@@ -89,6 +90,7 @@ void sweep_species(CasimDyad *d, double dt) {
     const int ly = layout_id(p);
     if (DIM == 3 && ly == 1) return sweep_slots<T, DIM, 1, 3, 3, 1, 1>(d, dt);
     if (ly == 2) return sweep_slots<T, DIM, 1, 3, 4, 0, 2>(d, dt);
+    if (ly == 3) return sweep_slots<T, DIM, 2, 4, 6, 0, 3>(d, dt);
     if (p.ni == 2 && p.nb == 4 && p.n_grid == 6 && p.n_face == 0) return sweep_slots<T, DIM, 2, 4, 6, 0, 0>(d, dt);
     return sweep_slots<T, DIM, 0, 0, 0, 0, 0>(d, dt);
 }
