@@ -147,6 +147,16 @@ void CasimDyad::sync() {
     casim::resident_check(this);
 }
 
+double *CasimDyad::pinned() {
+    if (!pin) {
+        HIPCK(hipHostMalloc((void **)&pin, sizeof(double) * PIN, hipHostMallocDefault));
+        HIPCK(hipEventCreateWithFlags(&pin_busy, hipEventDisableTiming));
+    } else {
+        HIPCK(hipEventSynchronize(pin_busy));
+    }
+    return pin;
+}
+
 void CasimDyad::launch_step(double dt) {
     if (precision == CASIM_FP64)
         step_dispatch<double>(this, dt);
@@ -196,7 +206,7 @@ void CasimDyad::launch_channels(int mode, double dt) {
 }
 
 void CasimDyad::launch_rim(const double *ions, const double *bound) {
-    dim3 grid((P.NS + 255) / 256, P.S);
+    dim3 grid((2 * (P.nx + P.ny - 2) * P.nz + 255) / 256, P.S);
     if (precision == CASIM_FP64)
         hipLaunchKernelGGL(k_rim<double>, grid, dim3(256), 0, stream, (double *)g[0], (double *)g[1],
                            (double *)f[0], (double *)f[1], ions, bound, P);
@@ -380,7 +390,12 @@ int casim_dyad_create(const CasimDyadConfig *c, CasimDyad **out) {
             const int th = Pl > 256 ? 256 : (Pl + 63) / 64 * 64;
             if (Pl <= 4 * 512 && lds <= 65536 && (Pl + th - 1) / th <= 4) {
                 d->sweep_threads = th;
-                d->sweep_chunk = P.nx - 2;
+                // enough chunks of planes for about four workgroups per CU: a whole
+                // site per workgroup marches its planes one after another with most
+                // CUs idle (128 sites of 61x61x5: 24 us per step, 71 whole); at least four
+                // planes, against the planes that neighbouring chunks load twice
+                const int inner = P.nx - 2, chunks = std::min((inner + 3) / 4, (1024 + P.S - 1) / P.S);
+                d->sweep_chunk = (inner + chunks - 1) / chunks;
             }
         }
 
@@ -488,14 +503,15 @@ int casim_dyad_create(const CasimDyadConfig *c, CasimDyad **out) {
         d->d_rng0 = dalloc<uint32_t>((size_t)P.S * 6);
         d->d_jump = dalloc<uint32_t>(jump.size());
         d->d_mouths = dalloc<double>((size_t)K * P.S * std::max(1, d->M));
-        d->d_jsr = dalloc<double>((size_t)P.ni * P.S * std::max(1, d->M));
         d->d_sJ = dalloc<double>((size_t)P.ni * std::max(1, d->nch));
         d->d_snap = dalloc<double>((size_t)(P.n_grid + P.n_face) * std::max(1, d->nch));
         d->d_pg = dalloc<double>((size_t)P.ni * std::max(1, d->nch));
         d->d_pjv = dalloc<double>((size_t)P.ni * std::max(1, d->nch));
         d->d_totals = dalloc<double>((size_t)P.ni * P.S);
-        d->d_rim_ions = dalloc<double>((size_t)P.ni * P.S);
-        d->d_rim_bound = dalloc<double>((size_t)std::max(1, P.nb) * P.S);
+        // the update's inputs in a row, so that one copy brings them
+        d->d_rim_ions = dalloc<double>((size_t)(P.ni + P.nb + P.ni * std::max(1, d->M)) * P.S);
+        d->d_rim_bound = d->d_rim_ions + (size_t)P.ni * P.S;
+        d->d_jsr = d->d_rim_bound + (size_t)P.nb * P.S;
         d->d_eff = dalloc<double>((size_t)(P.ni + P.nb) * P.S);
         d->d_stats = dalloc<double>((size_t)NSTAT * P.S);
         auto up = [&](void *dst, const void *src, size_t bytes) {
@@ -554,9 +570,11 @@ int casim_dyad_destroy(CasimDyad *d) {
     casim::box_free(d);
     casim::resident_free(d);
     casim::site2d_free(d);
+    if (d->pin) (void)hipHostFree(d->pin);
+    if (d->pin_busy) (void)hipEventDestroy(d->pin_busy);
     void *ptrs[] = {d->g[0], d->g[1], d->f[0], d->f[1], d->d_off, d->d_node, d->d_type, d->d_perm, d->d_snode,
-                    d->d_sperm, d->d_state, d->d_chans, d->d_rng, d->d_rng0, d->d_jump, d->d_mouths, d->d_jsr, d->d_sJ,
-                    d->d_snap, d->d_pg, d->d_pjv, d->d_totals, d->d_rim_ions, d->d_rim_bound, d->d_eff, d->d_stats, d->Ch.trace};
+                    d->d_sperm, d->d_state, d->d_chans, d->d_rng, d->d_rng0, d->d_jump, d->d_mouths, d->d_sJ,
+                    d->d_snap, d->d_pg, d->d_pjv, d->d_totals, d->d_rim_ions, d->d_eff, d->d_stats, d->Ch.trace};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (double *p : d->pool_buffers)
@@ -638,15 +656,24 @@ int casim_dyad_update(CasimDyad *d, const double *rim_ions, const double *rim_bo
         d->use();
         const Params &P = d->P;
         d->voltage = voltage;
-        if (!pool_rim && !box_rim) {
-            HIPCK(hipMemcpyAsync(d->d_rim_ions, rim_ions, sizeof(double) * P.ni * P.S, hipMemcpyHostToDevice,
-                                 d->stream));
-            if (P.nb)
-                HIPCK(hipMemcpyAsync(d->d_rim_bound, rim_bound, sizeof(double) * P.nb * P.S, hipMemcpyHostToDevice,
-                                     d->stream));
+        const bool rim = !pool_rim && !box_rim, chan = !d->Q.on && d->M;
+        const size_t ni = (size_t)P.ni * P.S, nb = (size_t)P.nb * P.S, nj = ni * d->M;
+        const bool staged = rim && chan && ni + nb + nj <= CasimDyad::PIN;
+        if (staged) {
+            std::lock_guard<std::mutex> lock(d->pin_mutex);
+            double *h = d->pinned();
+            std::memcpy(h, rim_ions, sizeof(double) * ni);
+            if (nb) std::memcpy(h + ni, rim_bound, sizeof(double) * nb);
+            std::memcpy(h + ni + nb, jsr, sizeof(double) * nj);
+            HIPCK(hipMemcpyAsync(d->d_rim_ions, h, sizeof(double) * (ni + nb + nj), hipMemcpyHostToDevice, d->stream));
+            HIPCK(hipEventRecord(d->pin_busy, d->stream));
+        } else {
+            if (rim) {
+                HIPCK(hipMemcpyAsync(d->d_rim_ions, rim_ions, sizeof(double) * ni, hipMemcpyHostToDevice, d->stream));
+                if (nb) HIPCK(hipMemcpyAsync(d->d_rim_bound, rim_bound, sizeof(double) * nb, hipMemcpyHostToDevice, d->stream));
+            }
+            if (chan) HIPCK(hipMemcpyAsync(d->d_jsr, jsr, sizeof(double) * nj, hipMemcpyHostToDevice, d->stream));
         }
-        if (!d->Q.on && d->M)
-            HIPCK(hipMemcpyAsync(d->d_jsr, jsr, sizeof(double) * P.ni * P.S * d->M, hipMemcpyHostToDevice, d->stream));
         if (pool_rim)
             d->launch_rim(d->Q.cions, d->Q.cbb);
         else if (box_rim)
@@ -656,7 +683,8 @@ int casim_dyad_update(CasimDyad *d, const double *rim_ions, const double *rim_bo
         d->launch_efflux();
         d->launch_channels(CH_SNAPSHOT | CH_CURRENTS | CH_ACCUMULATE | CH_POOL_UPDATE, 0.0);
         d->clear_graphs();
-        HIPCK(hipStreamSynchronize(d->stream));
+        // the caller's arrays are free: copied to the pinned buffer, or by now to the device
+        if (!staged) HIPCK(hipStreamSynchronize(d->stream));
         d->have_update = true;
     });
 }
@@ -665,6 +693,14 @@ int casim_dyad_update(CasimDyad *d, const double *rim_ions, const double *rim_bo
 
 namespace {
 void copy_out(CasimDyad *d, double *out, const double *src, size_t n) {
+    if (n <= CasimDyad::PIN) {
+        std::lock_guard<std::mutex> lock(d->pin_mutex);
+        double *h = d->pinned();
+        HIPCK(hipMemcpyAsync(h, src, sizeof(double) * n, hipMemcpyDeviceToHost, d->stream));
+        d->sync();
+        std::memcpy(out, h, sizeof(double) * n);
+        return;
+    }
     HIPCK(hipMemcpyAsync(out, src, sizeof(double) * n, hipMemcpyDeviceToHost, d->stream));
     d->sync();
 }
@@ -813,8 +849,7 @@ int casim_dyad_run_rd(CasimDyad *d, double dt, int32_t site) {
         REQUIRE(d->have_update, CASIM_E_STATE, "run_rd before the first update");
         REQUIRE(!d->box, CASIM_E_STATE, "with a cytosol box, advance with casim_dyad_step");
         d->use();
-        d->launch_step(dt);
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->launch_step(dt);  // what reads the state waits for the stream
     });
 }
 
@@ -825,7 +860,6 @@ int casim_dyad_run_mc(CasimDyad *d, double dt, int32_t site) {
         REQUIRE(d->have_update, CASIM_E_STATE, "run_mc before the first update");
         d->use();
         d->launch_channels(CH_GATE_STORED, dt);
-        HIPCK(hipStreamSynchronize(d->stream));
     });
 }
 

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <tuple>
@@ -97,6 +98,14 @@ struct CasimDyad {
     casim::Resident *res = nullptr;  // made by the first step that it can take
     bool res_tried = false;
     casim::Site2D *s2d = nullptr;
+    // Pinned buffer for small transfers (the update's inputs, site values): a
+    // copy from or to pageable memory is staged by the runtime, which waits for
+    // it.  pinned(): the buffer, free for use, with pin_mutex held.
+    static constexpr size_t PIN = (size_t)1 << 17;  // doubles
+    double *pin = nullptr;
+    hipEvent_t pin_busy = nullptr;
+    std::mutex pin_mutex;
+    double *pinned();
     // the sites and stream the pair and channel launchers work on (all sites
     // on `stream` unless casim_dyad_step splits the batch)
     int range_s0 = 0, range_n = -1;
