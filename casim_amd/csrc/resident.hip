@@ -4,7 +4,7 @@
 // HBM moves the state once per call instead of once per two steps, and a step
 // costs no launch.
 //
-// A slab is one workgroup on one CU: up to seven waves hold one node column
+// A slab is one workgroup on one CU: up to nine waves hold one node column
 // each lane (PL planes of three fields in registers), one more wave runs the
 // channels.  A step is a row of phases between barriers: first the slab's two
 // edge planes, so that the neighbours get them a step ahead of their use, then
@@ -140,8 +140,10 @@ __device__ __forceinline__ bool wait_flags(const unsigned *watch, unsigned targe
 }
 
 // ---------------------------------------------------------------------------
+// waves of a workgroup for planes of PS nodes, and per SIMD
+constexpr int res_waves(int PS) { return (PS + 63) / 64 + 1; }
 template <typename T, int PL, int PH, int PS>
-__global__ __launch_bounds__((PS + 63) / 64 * 64 + 64, 2) void k_resident(const T *__restrict__ gin,
+__global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k_resident(const T *__restrict__ gin,
                                                                             T *__restrict__ gout,
                                                                             const T *__restrict__ fin,
                                                                             T *__restrict__ fout, const Params p,
@@ -801,6 +803,10 @@ const Form FORMS[] = {
     form<double, 20, 4, 440>(2.1, 0.37), form<double, 10, 3, 440>(2.1, 0.37), form<double, 5, 3, 440>(2.1, 0.37),
     form<float, 40, 8, 440>(2.0, 0.25),  form<float, 20, 6, 440>(2.0, 0.25),  form<float, 10, 3, 440>(2.0, 0.25),
     form<float, 5, 3, 440>(2.0, 0.25),
+    // three waves per SIMD, 168 registers (81x96x6, 100 steps, ms, the sweeps before: 32 sites 15.2 -> 1.1,
+    // 200 sites 17.5 -> 7.1, FP32 2500 sites 41.6 -> 30.7; FP64 2500 sites 73.5, 79.8 here, so by the sweeps)
+    form<double, 10, 3, 576>(0.6, 0.94), form<double, 5, 3, 576>(0.6, 0.94), form<float, 20, 6, 576>(3.7, 0.18),
+    form<float, 10, 3, 576>(3.7, 0.18),  form<float, 5, 3, 576>(3.7, 0.18),
 };
 
 }  // namespace
