@@ -190,7 +190,9 @@ void box_set_cur(CasimDyad *d, int cur);
 struct CasimMLP;
 namespace casim {
 // Device-side ensemble forward (mlp.hip): out [members x rows], normalised units.
-void mlp_forward_device(CasimMLP *m, const float *x, int64_t rows, float *out, hipStream_t stream);
+void mlp_forward_device(CasimMLP *m, const float *x, int64_t rows, float *out, int64_t ostride, const int *rows_d,
+                        hipStream_t stream);
+bool mlp_rows_on_device(const CasimMLP *m);
 int mlp_members(const CasimMLP *m);
 int mlp_inputs(const CasimMLP *m);
 float mlp_out_mean(const CasimMLP *m);

@@ -191,6 +191,7 @@ struct InferArgs {
     int wtoff[IMAXL], boff[IMAXL], kp[IMAXL], fout[IMAXL];
     int nl, n_in;
     const float *mean, *istd;
+    const int *rows_d;  // rows of this call, where only the device knows them (or null)
 };
 
 // Place of element (n, k) of a [n][k] operand with nk blocks of 32 in k, in the
@@ -228,6 +229,8 @@ __global__ __launch_bounds__(64 * IWAVES / CT, 4) void k_mlp_infer(const float *
     __shared__ __attribute__((aligned(16))) uint16_t H[2][R][IMAXW + IPADK];
     const int m0 = blockIdx.x * R, e = blockIdx.y;
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
+    if (a.rows_d) rows = min(rows, *a.rows_d);
+    if (m0 >= rows) return;
     const uint16_t *wt = a.wt[e];
     const float *pe = a.p[e];
     // every k-block of the wave's columns for layer L, and their biases, issued
@@ -762,7 +765,7 @@ struct CasimMLP {
     bool fused_ok() const;
     size_t wt_offsets(int *off) const;
     void refresh_wt();
-    void infer(const float *x, int B, float *out, int ostride);
+    void infer(const float *x, int B, float *out, int ostride, const int *rows_d = nullptr);
     // batch workspace
     int cap = 0;
     std::vector<uint16_t *> Xl;  // [depth + 1] BF16 activations
@@ -845,7 +848,7 @@ void CasimMLP::refresh_wt() {
 }
 
 // Every member's output (normalised units) for B raw rows x -> out[e * ostride + row].
-void CasimMLP::infer(const float *x, int B, float *out, int ostride) {
+void CasimMLP::infer(const float *x, int B, float *out, int ostride, const int *rows_d) {
     refresh_wt();
     InferArgs a{};
     int off[2 * IMAXL];
@@ -864,6 +867,7 @@ void CasimMLP::infer(const float *x, int B, float *out, int ostride) {
     a.n_in = n_in;
     a.mean = mean;
     a.istd = istd;
+    a.rows_d = rows_d;
     const int big = (B + 63) / 64;
     if ((size_t)big * members >= INFER_BIG)
         hipLaunchKernelGGL((k_mlp_infer<2, 4>), dim3((unsigned)big, (unsigned)members), dim3(32 * IWAVES), 0, stream, x, B, out,
@@ -1097,31 +1101,33 @@ void CasimMLP::train_group(int e0, int mg, int epochs, int B, float lr, uint64_t
 namespace casim {
 
 // Every member's output (normalised units) for `rows` raw feature rows on the
-// device: x [rows x n_in] -> out [members x rows].  Runs on `stream` after
-// the MLP's own stream has drained.
-void mlp_forward_device(CasimMLP *m, const float *x, int64_t rows, float *out, hipStream_t stream) {
+// device: x [rows x n_in] -> out [members x ostride].  Runs on `stream` after
+// the MLP's own stream has drained.  rows_d: the number of rows in device
+// memory, at most `rows`; only with mlp_rows_on_device.
+void mlp_forward_device(CasimMLP *m, const float *x, int64_t rows, float *out, int64_t ostride, const int *rows_d,
+                        hipStream_t stream) {
     m->use();
     HIPCK(hipStreamSynchronize(m->stream));
     hipStream_t keep = m->stream;
     m->stream = stream;
     try {
-        const int chunk = (int)std::min<int64_t>(rows, 65536);
-        if (!m->fused_ok()) m->reserve(chunk);
-        for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
-            const int B = (int)std::min<int64_t>(chunk, rows - r0);
-            if (m->fused_ok()) {
-                m->infer(x + r0 * m->n_in, B, out + r0, (int)rows);
-                continue;
-            }
-            const size_t n = (size_t)B * m->n_in;
-            hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                               x + r0 * m->n_in, (const float *)nullptr, (const int *)nullptr, B, m->n_in, m->mean,
-                               m->istd, 0.f, 1.f, m->Xl[0], (float *)nullptr);
-            HIPCK(hipGetLastError());
-            for (int e = 0; e < m->members; ++e) {
-                m->forward(e, B);
-                HIPCK(hipMemcpyAsync(out + (size_t)e * rows + r0, m->Zl[m->depth], sizeof(float) * B,
-                                     hipMemcpyDeviceToDevice, stream));
+        if (m->fused_ok()) {
+            m->infer(x, (int)rows, out, (int)ostride, rows_d);
+        } else {
+            const int chunk = (int)std::min<int64_t>(rows, 65536);
+            m->reserve(chunk);
+            for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
+                const int B = (int)std::min<int64_t>(chunk, rows - r0);
+                const size_t n = (size_t)B * m->n_in;
+                hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x + r0 * m->n_in,
+                                   (const float *)nullptr, (const int *)nullptr, B, m->n_in, m->mean, m->istd, 0.f, 1.f,
+                                   m->Xl[0], (float *)nullptr);
+                HIPCK(hipGetLastError());
+                for (int e = 0; e < m->members; ++e) {
+                    m->forward(e, B);
+                    HIPCK(hipMemcpyAsync(out + (size_t)e * ostride + r0, m->Zl[m->depth], sizeof(float) * B,
+                                         hipMemcpyDeviceToDevice, stream));
+                }
             }
         }
     } catch (...) {
@@ -1131,6 +1137,7 @@ void mlp_forward_device(CasimMLP *m, const float *x, int64_t rows, float *out, h
     m->stream = keep;
 }
 
+bool mlp_rows_on_device(const CasimMLP *m) { return m->fused_ok(); }
 int mlp_members(const CasimMLP *m) { return m->members; }
 int mlp_inputs(const CasimMLP *m) { return m->n_in; }
 float mlp_out_mean(const CasimMLP *m) { return m->ym; }

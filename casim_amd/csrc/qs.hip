@@ -43,7 +43,8 @@ struct QsDev {
     int *cur_bin;    // [S] first bin not yet written
     double bin_ms;
     int bins;
-    int R;         // surrogate rows this round (member stride of out)
+    int R;         // member stride of out
+    const int *cnt;  // this round's counts (k_qs_plan)
     double *stats;
     double *jsr;      // [S] current jSR
     double *jsr_min;  // [S] lowest jSR over [0, t_max]
@@ -148,6 +149,7 @@ __global__ __launch_bounds__(64 * QS_FWAVES) void k_qs_features(QsDev q) {
     __shared__ int so[QS_MAXCH], ol[QS_MAXCH];
     __shared__ int s_nopen;
     __shared__ __attribute__((aligned(16))) float part[QS_FWAVES - 1][64 * QS_PSTRIDE];
+    if ((int)blockIdx.x >= q.cnt[3]) return;
     const int s = q.list[blockIdx.x];  // one workgroup per site with rows this round
     const int base = q.crow[s];
     if (base < 0) return;
@@ -276,17 +278,33 @@ __device__ double jsr_advance(const QsDev &q, double c, double geff, double dt) 
 // event per site unless the surrogate is too uncertain for it: the site asks
 // for the full solver when the rate-weighted mean of the relative spreads,
 // sum_i (rate_i / total) spread_i, exceeds the threshold.
-__global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
+//
+// A latency chain: two waves take the channels, a third draws meanwhile.
+constexpr int QS_ETHREADS = QS_MAXCH + 64;
+__global__ __launch_bounds__(QS_ETHREADS) void k_qs_event(QsDev q) {
     __shared__ double rate[QS_MAXCH], wv[QS_MAXCH], pcv[QS_MAXCH];
     __shared__ float spv[QS_MAXCH], cav[QS_MAXCH];
-    __shared__ double s_total;
+    __shared__ double s_total, s_u[2];
+    __shared__ uint32_t s_rng[6];
+    if ((int)blockIdx.x >= q.cnt[3]) return;
     const int s = q.list[blockIdx.x];  // one workgroup per site with rows this round
     const int lane = threadIdx.x;
     const int base = q.crow[s];
     if (base < 0) return;
     const int off = q.off[s], n = q.off[s + 1] - off;
     const int wait = q.waiting[s];
-    for (int i = lane; i < n; i += 64) {
+    if (lane == QS_MAXCH) {
+        // Gillespie step (QuasyStationaryReleaseSite.cpp:101-128): waiting time,
+        // channel, MakeTransition(runif()); kept only if the site takes the event
+        uint32_t S6[6];
+        for (int k = 0; k < 6; ++k) S6[k] = q.rng[s * 6 + k];
+        const double u1 = mrg::draw(S6);
+        s_u[1] = mrg::draw(S6);
+        (void)mrg::draw(S6);
+        s_u[0] = -log(u1);
+        for (int k = 0; k < 6; ++k) s_rng[k] = S6[k];
+    }
+    for (int i = lane; i < n; i += QS_ETHREADS) {
         const size_t row = off + i;
         float ca, sp;
         if (q.st_n > 0) {
@@ -326,22 +344,23 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
     // on all lanes (the serial sums below then only add)
     if (lane == 0) {
         double tot = 0.0;
+#pragma unroll 8
         for (int i = 0; i < n; ++i) tot += rate[i];
         s_total = tot;
     }
     __syncthreads();
     const double total = s_total;
     if (total > 0.0)
-        for (int i = lane; i < n; i += 64) wv[i] = rate[i] / total;
+        for (int i = lane; i < n; i += QS_ETHREADS) wv[i] = rate[i] / total;
     __syncthreads();
+    if (lane >= 64) return;
     double *st = q.stats + (size_t)s * QS_NSTAT;
     // lane 0: the shares' running sums in channel order (pcv[i], the sum of
     // the shares before channel i), the spread test and the event's draws;
     // then every lane tests its channels against the draw and a ballot finds
     // the first one, the channel the serial scan would stop at
     int go = 0;
-    double u1 = 0.0, r = 0.0;
-    uint32_t S6[6];
+    const double r = s_u[1];
     if (lane == 0) {
         if (!(total > 0.0)) {
             // nothing can happen any more: N stays until t_max, and the open
@@ -360,6 +379,7 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
             q.waiting[s] = 0;
         } else {
             double pc = 0.0, m = 0.0;
+#pragma unroll 8
             for (int i = 0; i < n; ++i) {
                 pcv[i] = pc;
                 m += wv[i] * (double)spv[i];
@@ -369,17 +389,12 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
                 q.waiting[s] = 1;
             } else {
                 q.waiting[s] = 0;
-                // Gillespie step (QuasyStationaryReleaseSite.cpp:101-128)
-                for (int k = 0; k < 6; ++k) S6[k] = q.rng[s * 6 + k];
-                u1 = mrg::draw(S6);
-                r = mrg::draw(S6);
                 go = 1;
             }
         }
     }
     go = __shfl(go, 0);
     if (!go) return;  // the whole wave
-    r = __shfl(r, 0);
     __syncthreads();
     int idx = 0;
     {
@@ -390,8 +405,8 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
         if (b0) idx = __ffsll((long long)b0) - 1;
         else if (b1) idx = 64 + __ffsll((long long)b1) - 1;
     }
-    double dtw = 0.0, cw = 0.0;
-    if (lane == 0) dtw = -log(u1) * (1.0 / total);
+    const double dtw = s_u[0] * (1.0 / total);
+    double cw = 0.0;
     if (q.deplete) {
         // the jSR over the interval before the event, with this interval's open
         // set: every channel's share of the conductance on its lane, summed in
@@ -399,9 +414,9 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
         const double c0 = q.jsr[s], tmax = q.t_max - q.t[s];
         for (int i = lane; i < n; i += 64) pcv[i] = q.state[off + i] == 1 ? q.gch * (1.0 - (double)cav[i] / c0) : 0.0;
         __syncthreads();
-        dtw = __shfl(dtw, 0);
         if (lane > 1) return;
         double geff = 0.0;
+#pragma unroll 8
         for (int i = 0; i < n; ++i) geff += pcv[i];
         // lane 1 meanwhile goes to t_max where the event lies past it: the lowest
         // jSR over [0, t_max] is what a run of that length observes
@@ -416,7 +431,6 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
     }
     if (lane != 0) return;
     const double t = q.t[s] + dtw;
-    (void)mrg::draw(S6);  // MakeTransition(runif())
     if (q.trace) {
         // IndChannelCREAnalyzer.cpp:78-84: bins up to the next record's time
         // take the current count
@@ -447,7 +461,7 @@ __global__ __launch_bounds__(64) void k_qs_event(QsDev q) {
     st[QS_NCUR] = nnew;
     st[QS_EVENTS] += 1.0;
     q.t[s] = t;
-    for (int k = 0; k < 6; ++k) q.rng[s * 6 + k] = S6[k];
+    for (int k = 0; k < 6; ++k) q.rng[s * 6 + k] = s_rng[k];
     if (nnew < 1.0 || t >= q.t_max) q.active[s] = 0;
 }
 
@@ -479,9 +493,14 @@ __global__ void k_qs_init(QsDev q, const int *__restrict__ init, const uint32_t 
 }
 
 // Rows of this round: every site with `all`, else the active sites that do
-// not wait for the full solver, packed in site order (one block).  cnt[0..2]:
-// active sites, waiting sites, rows.
-__global__ __launch_bounds__(1024) void k_qs_plan(QsDev q, int all, int *__restrict__ cnt) {
+// not wait for the full solver, packed in site order (one block).  cnt: active
+// sites, waiting sites, rows, sites with rows, rounds taken since the first
+// plan of a run; a copy goes to the host's memory.  Without a next round (no
+// site left, or `batch` sites waiting, or all of them) there are no rows and the
+// kernels of a round have nothing to do, so the host enqueues several rounds
+// and looks once.
+__global__ __launch_bounds__(1024) void k_qs_plan(QsDev q, int all, int first, int batch, int *__restrict__ cnt,
+                                                  int *__restrict__ host) {
     // per-wave totals of the four counts, then their running sums (16 waves)
     __shared__ int wsum[4][16], wpre[4][16];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -530,10 +549,12 @@ __global__ __launch_bounds__(1024) void k_qs_plan(QsDev q, int all, int *__restr
         }
     }
     if (t == 1023) {
-        cnt[0] = wpre[2][15] + v[2];
-        cnt[1] = wpre[3][15] + v[3];
-        cnt[2] = wpre[0][15] + v[0];
-        cnt[3] = wpre[1][15] + v[1];  // sites with rows: the grid of k_qs_features and k_qs_event
+        const int act = wpre[2][15] + v[2], wt = wpre[3][15] + v[3];
+        const bool go = all || (act > 0 && wt < batch && wt < act);
+        const int c5[5] = {act, wt, go ? wpre[0][15] + v[0] : 0, go ? wpre[1][15] + v[1] : 0,
+                           first ? 0 : cnt[4] + (cnt[3] > 0)};
+#pragma unroll
+        for (int k = 0; k < 5; ++k) cnt[k] = host[k] = c5[k];
     }
 }
 
@@ -546,7 +567,7 @@ struct CasimQS {
     int nch = 0;
     std::vector<int> h_off, h_init;
     std::vector<uint32_t> h_rng0;
-    int *d_init = nullptr, *d_count = nullptr;
+    int *d_init = nullptr, *d_count = nullptr, *h_count = nullptr;  // h_count: in the host's memory
     double *d_jsr0 = nullptr;
     uint32_t *d_rng0 = nullptr, *d_jump = nullptr;
     std::vector<void *> bufs;
@@ -678,7 +699,11 @@ int casim_qs_create(const CasimQSConfig *c, CasimQS **out) {
         q.gch = c->conductance;
         q.thresh = (float)c->spread_threshold;
         h->d_init = h->alloc<int>(S);
-        h->d_count = h->alloc<int>(4);
+        h->d_count = h->alloc<int>(5);
+        HIPCK(hipMemsetAsync(h->d_count, 0, sizeof(int) * 5, h->stream));
+        HIPCK(hipHostMalloc((void **)&h->h_count, sizeof(int) * 8, hipHostMallocMapped));
+        q.cnt = h->d_count;
+        q.R = h->nch;
         q.cur_bin = h->alloc<int>(S);
         q.trace = nullptr;
         q.bins = 0;
@@ -713,6 +738,7 @@ int casim_qs_destroy(CasimQS *h) {
     if (h->q.out) (void)hipFree(h->q.out);
     if (h->q.trace) (void)hipFree(h->q.trace);
     if (h->q.lin_tab) (void)hipFree((void *)h->q.lin_tab);
+    if (h->h_count) (void)hipHostFree(h->h_count);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
     return CASIM_OK;
@@ -752,26 +778,33 @@ int casim_qs_run(CasimQS *h, CasimMLP *m, int32_t max_rounds, int32_t wait_batch
             h->q.ys = mlp_out_std(m);
         }
         const int batch = std::max(1, (int)wait_batch);
-        int cnt[4] = {0, 0, 0, 0};
-        auto plan = [&] {
-            hipLaunchKernelGGL(k_qs_plan, dim3(1), dim3(1024), 0, h->stream, h->q, 0, h->d_count);
+        volatile int *cnt = h->h_count;
+        auto plan = [&](int first) {
+            hipLaunchKernelGGL(k_qs_plan, dim3(1), dim3(1024), 0, h->stream, h->q, 0, first, batch, h->d_count, h->h_count);
             HIPCK(hipGetLastError());
-            HIPCK(hipMemcpyAsync(cnt, h->d_count, sizeof(int) * 4, hipMemcpyDeviceToHost, h->stream));
-            HIPCK(hipStreamSynchronize(h->stream));
         };
-        plan();
+        plan(1);
+        HIPCK(hipStreamSynchronize(h->stream));
         int r = 0;
         while (r < max_rounds && cnt[0] > 0 && cnt[1] < batch && cnt[1] < cnt[0]) {
-            h->q.R = cnt[2];
-            if (!stationary) {
-                hipLaunchKernelGGL(k_qs_features, dim3(cnt[3]), dim3(64 * QS_FWAVES), 0, h->stream, h->q);
+            // rounds enqueued at a time: the counts only shrink, so the last ones
+            // known bound the grids; many rows make the wait small and empty
+            // workgroups dear.  Without the fused kernel the host has to know the rows.
+            const int rows = cnt[2], sites = cnt[3];
+            const int most = !stationary && !mlp_rows_on_device(m) ? 1 : rows > 32768 ? 1 : rows > 4096 ? 4 : 8;
+            const int k = std::min(most, (int)max_rounds - r);
+            for (int i = 0; i < k; ++i) {
+                if (!stationary) {
+                    hipLaunchKernelGGL(k_qs_features, dim3(sites), dim3(64 * QS_FWAVES), 0, h->stream, h->q);
+                    HIPCK(hipGetLastError());
+                    mlp_forward_device(m, h->q.X, rows, h->q.out, h->nch, k > 1 ? h->d_count + 2 : nullptr, h->stream);
+                }
+                hipLaunchKernelGGL(k_qs_event, dim3(sites), dim3(QS_ETHREADS), 0, h->stream, h->q);
                 HIPCK(hipGetLastError());
-                mlp_forward_device(m, h->q.X, cnt[2], h->q.out, h->stream);
+                plan(0);
             }
-            hipLaunchKernelGGL(k_qs_event, dim3(cnt[3]), dim3(64), 0, h->stream, h->q);
-            HIPCK(hipGetLastError());
-            ++r;
-            plan();
+            HIPCK(hipStreamSynchronize(h->stream));
+            r = cnt[4];
         }
         if (rounds) *rounds = r;
         if (n_active) *n_active = cnt[0];
@@ -939,7 +972,7 @@ int casim_qs_get_features(CasimQS *h, float *out) {
     return guard([&] {
         REQUIRE(h && out, CASIM_E_INVALID, "null argument");
         h->use();
-        hipLaunchKernelGGL(k_qs_plan, dim3(1), dim3(1024), 0, h->stream, h->q, 1, h->d_count);
+        hipLaunchKernelGGL(k_qs_plan, dim3(1), dim3(1024), 0, h->stream, h->q, 1, 1, 0, h->d_count, h->h_count);
         HIPCK(hipGetLastError());
         hipLaunchKernelGGL(k_qs_features, dim3(h->q.S), dim3(64 * QS_FWAVES), 0, h->stream, h->q);
         HIPCK(hipGetLastError());
