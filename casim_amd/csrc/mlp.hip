@@ -125,18 +125,27 @@ __global__ __launch_bounds__(256) void k_gemm(const uint16_t *__restrict__ A, in
 
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.f / (1.f + __expf(-z)); }
 
-// sigmoidf_ of four values.  1 / d for 1 <= d <= 2^125 by the hardware's
+// sigmoidf_ of N values.  1 / d for 1 <= d <= 2^125 by the hardware's
 // reciprocal and one Newton step, which gives the correctly rounded quotient,
 // the compiler's result, for every float in that range (compared one by one);
 // its general division takes 11 operations.  Below -86 the general one.
-__device__ __forceinline__ void sigmoid4(const float (&z)[4], float (&s)[4]) {
-    if (fminf(fminf(z[0], z[1]), fminf(z[2], z[3])) < -86.f) {
+template <int N>
+__device__ __forceinline__ void sigmoid_n(const float (&z)[N], float (&s)[N]) {
+    float lo = z[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[i] = sigmoidf_(z[i]);
+    for (int i = 1; i < N; ++i) lo = __builtin_fminf(lo, z[i]);
+    if (lo < -86.f) {
+#pragma unroll 1
+        for (int i = 0; i < N; i += 4)
+#pragma unroll
+            for (int k = 0; k < N; k += 4)
+                if (k == i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[k + r] = sigmoidf_(z[k + r]);
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < N; ++i) {
         const float d = 1.f + __expf(-z[i]), y = __builtin_amdgcn_rcpf(d);
         s[i] = __builtin_fmaf(__builtin_fmaf(-d, y, 1.f), y, y);
     }
@@ -145,10 +154,13 @@ __device__ __forceinline__ void sigmoid4(const float (&z)[4], float (&s)[4]) {
 // f2bf of four values by the conversion instruction (two values each, the same
 // rounding)
 __device__ __forceinline__ void f2bf4(const float (&f)[4], uint16_t (&h)[4]) {
-    __bf16 b[4];
+    typedef float __attribute__((ext_vector_type(2))) f2_t;
+    typedef __bf16 __attribute__((ext_vector_type(2))) b2_t;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) b[i] = (__bf16)f[i];
-    std::memcpy(h, b, sizeof h);
+    for (int i = 0; i < 4; i += 2) {
+        const b2_t b = __builtin_convertvector((f2_t{f[i], f[i + 1]}), b2_t);
+        std::memcpy(h + i, &b, sizeof b);
+    }
 }
 
 // Z += b (per column); H = bf16(SiLU(Z)) or bf16(Z) for the last layer.
@@ -175,13 +187,13 @@ __global__ void k_bias_act(float *__restrict__ Z, const float *__restrict__ b, u
 // their way while a layer runs.  Many rows: eight waves with 32 columns each, 64
 // rows, two workgroups per CU.  The weights are then read half as often and the
 // rows' operands from LDS feed two products; what bounds it is the SiLU, about
-// 14 vector operations per activation (55003 rows: 249 us, 276 with the
-// compiler's division in it, 25 operations).  Times in us for five members of width
+// 14 vector operations per activation (276 us with the compiler's division in
+// it, 25 operations).  Times in us for five members of width
 // 256, depth 4 (before: weights in plain rows, 32 rows per workgroup):
 //   rows        512   2048   4096   8192   16384   55003
 //   before       -      -      -      -      195     658
-//   32 rows      17     29     42     66     126     424
-//   64 rows      26     28     39     55      86     276
+//   32 rows      15     26     42     66     126     424
+//   64 rows      26     28     32     50      78     240
 // so 64 rows from INFER_BIG workgroups on, one per CU.
 constexpr int IMR = 32, IMAXW = 256, IPADK = 8, IMAXM = 8, IMAXL = 8, IWAVES = IMAXW / 16;
 constexpr size_t INFER_BIG = 256;
@@ -226,6 +238,7 @@ template <int CT, int RT>
 __global__ __launch_bounds__(64 * IWAVES / CT, 4) void k_mlp_infer(const float *__restrict__ X, int rows,
                                                                    float *__restrict__ out, int ostride, InferArgs a) {
     constexpr int R = 16 * RT, NT = 64 * IWAVES / CT;
+    constexpr int GR = CT == 1 ? 2 : 1;  // row tiles whose activations are formed together, as registers allow
     __shared__ __attribute__((aligned(16))) uint16_t H[2][R][IMAXW + IPADK];
     const int m0 = blockIdx.x * R, e = blockIdx.y;
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
@@ -297,24 +310,28 @@ __global__ __launch_bounds__(64 * IWAVES / CT, 4) void k_mlp_infer(const float *
                 const int col = (w * CT + c) * 16 + (l & 15);
                 if (col >= N) break;
 #pragma unroll
-                for (int i = 0; i < RT; ++i) {
-                    const int row = i * 16 + (l >> 4) * 4;
-                    float z[4];
+                for (int i0 = 0; i0 < RT; i0 += GR) {
+                    const int row = i0 * 16 + (l >> 4) * 4;
+                    float z[4 * GR], sg[4 * GR];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) z[r] = acc[c][i][r] + b0[c];
+                    for (int i = 0; i < 4 * GR; ++i) z[i] = acc[c][i0 + i / 4][i % 4] + b0[c];
                     if (last) {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (m0 + row + r < rows) out[(size_t)e * ostride + m0 + row + r] = z[r];
+                        for (int i = 0; i < 4 * GR; ++i) {
+                            const int m = m0 + row + i / 4 * 16 + i % 4;
+                            if (m < rows) out[(size_t)e * ostride + m] = z[i];
+                        }
                     } else {
-                        float sg[4];
-                        uint16_t h[4];
-                        sigmoid4(z, sg);
+                        sigmoid_n(z, sg);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) z[r] *= sg[r];
-                        f2bf4(z, h);
+                        for (int i = 0; i < GR; ++i) {
+                            const float f[4] = {z[4 * i] * sg[4 * i], z[4 * i + 1] * sg[4 * i + 1],
+                                                z[4 * i + 2] * sg[4 * i + 2], z[4 * i + 3] * sg[4 * i + 3]};
+                            uint16_t h[4];
+                            f2bf4(f, h);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) H[src ^ 1][row + r][col] = h[r];
+                            for (int r = 0; r < 4; ++r) H[src ^ 1][row + 16 * i + r][col] = h[r];
+                        }
                     }
                 }
             }
@@ -533,7 +550,7 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
                 uint16_t h[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) zz[r] = z[r] = acc[i][r] + bias;
-                sigmoid4(z, f);
+                sigmoid_n(z, f);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) f[r] *= z[r];
                 f2bf4(f, h);
@@ -593,7 +610,7 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
                 const float z[4] = {zz[i][0], zz[i][1], zz[i][2], zz[i][3]};
                 float dz[4], sg[4];
                 uint16_t h[4];
-                sigmoid4(z, sg);
+                sigmoid_n(z, sg);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = i * 16 + rq + r;
@@ -780,9 +797,12 @@ struct CasimMLP {
     uint16_t *tr_x = nullptr, *tr_dzt = nullptr;
     float *tr_dz = nullptr, *tr_z = nullptr, *tr_sq = nullptr;
     int *tr_idx = nullptr;
-    // features and outputs of casim_mlp_predict, for pr_rows rows at a time
+    // features and outputs of casim_mlp_predict, two slots of pr_rows rows
     int pr_rows = 0;
     float *pr_x = nullptr, *pr_out = nullptr;
+    float *pr_pin = nullptr;          // the same in pinned memory
+    hipStream_t pr_stream = nullptr;  // its copies
+    hipEvent_t pr_up = nullptr, pr_done[2] = {};
     void predict_reserve(int b);
     bool train_fused(int B) const;
     int train_members(int B) const;
@@ -906,18 +926,28 @@ int CasimMLP::train_members(int B) const {
     return (int)std::min<size_t>(members, std::max<size_t>(1, ((size_t)1 << 30) / train_bytes(this, B)));
 }
 
-// Rows of a chunk of casim_mlp_predict, which bounds what a handle keeps for it.
-constexpr int PREDICT_ROWS = 65536;
+// Rows of a chunk of casim_mlp_predict, which bounds what a handle keeps for it;
+// enough to fill the chip (80 us of the ensemble kernel at five members).
+constexpr int PREDICT_ROWS = 16384;
 
 void CasimMLP::predict_reserve(int b) {
+    if (!pr_stream) {
+        HIPCK(hipStreamCreateWithFlags(&pr_stream, hipStreamNonBlocking));
+        for (hipEvent_t *e : {&pr_up, &pr_done[0], &pr_done[1]}) HIPCK(hipEventCreateWithFlags(e, hipEventDisableTiming));
+    }
     if (b <= pr_rows) return;
+    // whole powers of two, so that a caller whose batches grow does not allocate each time
+    int n = 256;
+    while (n < b) n *= 2;
     if (pr_x) (void)hipFree(pr_x);
     if (pr_out) (void)hipFree(pr_out);
-    pr_x = pr_out = nullptr;
+    if (pr_pin) (void)hipHostFree(pr_pin);
+    pr_x = pr_out = pr_pin = nullptr;
     pr_rows = 0;
-    HIPCK(hipMalloc(&pr_x, sizeof(float) * (size_t)b * n_in));
-    HIPCK(hipMalloc(&pr_out, sizeof(float) * (size_t)b * (members + 2)));
-    pr_rows = b;
+    HIPCK(hipMalloc(&pr_x, sizeof(float) * 2 * (size_t)n * n_in));
+    HIPCK(hipMalloc(&pr_out, sizeof(float) * 2 * (size_t)n * members));
+    HIPCK(hipHostMalloc((void **)&pr_pin, sizeof(float) * 2 * (size_t)n * (n_in + members + 2), hipHostMallocDefault));
+    pr_rows = n;
 }
 
 void CasimMLP::train_free() {
@@ -1192,18 +1222,18 @@ __global__ void k_na_collect(const float *__restrict__ z, float *__restrict__ ou
     if (r < rows) out[r] = z[r];
 }
 
-// Mean and relative spread of exp(y * ys + ym) over the members; with keep, out
-// becomes y * ys + ym.  A few us for 55003 rows of five members, where the same
-// sums on the host, member by member after a copy of its outputs, took 1 ms.
-__global__ void k_na_reduce(float *__restrict__ out, int members, int cap, int rows, float ys, float ym,
-                            float *__restrict__ mean, float *__restrict__ spread, int keep) {
+// Mean and relative spread of exp(y * ys + ym) over the members; raw (out, or
+// null: not wanted) receives y * ys + ym.  4 us for 55003 rows of five members;
+// on the host, member by member after a copy of its outputs, 1 ms.
+__global__ void k_na_reduce(const float *out, int members, int cap, int rows, float ys, float ym,
+                            float *__restrict__ mean, float *__restrict__ spread, float *raw, int rcap) {
 #pragma clang fp contract(off)
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     double s = 0, s2 = 0;
     for (int e = 0; e < members; ++e) {
         const float o = out[(size_t)e * cap + r] * ys + ym;
-        if (keep) out[(size_t)e * cap + r] = o;
+        if (raw) raw[(size_t)e * rcap + r] = o;
         const double v = exp((double)o);
         s += v;
         s2 += v * v;
@@ -1294,6 +1324,10 @@ int casim_mlp_destroy(CasimMLP *m) {
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     m->free_batch();
     m->train_free();
+    if (m->pr_stream) (void)hipStreamDestroy(m->pr_stream);
+    if (m->pr_pin) (void)hipHostFree(m->pr_pin);
+    for (hipEvent_t e : {m->pr_up, m->pr_done[0], m->pr_done[1]})
+        if (e) (void)hipEventDestroy(e);
     for (auto v : {&m->p, &m->g, &m->am, &m->av})
         for (float *q : *v) (void)hipFree(q);
     for (uint16_t *q : m->pb) (void)hipFree(q);
@@ -1464,40 +1498,60 @@ int casim_mlp_predict(CasimMLP *m, const float *x, int64_t rows, float *mean, fl
     return guard([&] {
         REQUIRE(m && x && rows >= 1, CASIM_E_INVALID, "bad arguments");
         m->use();
-        const int chunk = (int)std::min<int64_t>(rows, PREDICT_ROWS);
+        const int chunk = (int)std::min<int64_t>(rows, PREDICT_ROWS), E = m->members;
         const bool fused = m->fused_ok();
         if (!fused) m->reserve(chunk);
         m->predict_reserve(chunk);
-        const int B0 = m->pr_rows;  // row stride of the device outputs
-        float *const raw = m->pr_out, *const mu = raw + (size_t)m->members * B0, *const sd = mu + B0;
-        for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
+        // two slots: while a chunk is evaluated, the next one is copied to pinned
+        // memory and on to the device, and the outputs, which the kernel writes to
+        // pinned memory, go to the caller (five members, us: 55003 rows 530, 740 with
+        // one copy each from and to pageable memory; 100 rows 39, 150)
+        const int cap = m->pr_rows, nc = (int)((rows + chunk - 1) / chunk);
+        const size_t slot = (size_t)cap * (m->n_in + E + 2);
+        auto take = [&](int c) {
+            const int64_t r0 = (int64_t)c * chunk;
             const int B = (int)std::min<int64_t>(chunk, rows - r0);
-            HIPCK(hipMemcpyAsync(m->pr_x, x + r0 * m->n_in, sizeof(float) * (size_t)B * m->n_in, hipMemcpyHostToDevice,
-                                 m->stream));
+            const float *h = m->pr_pin + (c & 1) * slot + (size_t)cap * m->n_in;
+            HIPCK(hipEventSynchronize(m->pr_done[c & 1]));
+            for (int e = 0; member_out && e < E; ++e)
+                std::memcpy(member_out + (size_t)e * rows + r0, h + (size_t)e * B, sizeof(float) * B);
+            if (mean) std::memcpy(mean + r0, h + (size_t)E * B, sizeof(float) * B);
+            if (spread) std::memcpy(spread + r0, h + (size_t)(E + 1) * B, sizeof(float) * B);
+        };
+        for (int c = 0; c < nc; ++c) {
+            if (c >= 2) take(c - 2);
+            const int64_t r0 = (int64_t)c * chunk;
+            const int B = (int)std::min<int64_t>(chunk, rows - r0);
+            float *const hx = m->pr_pin + (c & 1) * slot, *const ho = hx + (size_t)cap * m->n_in;
+            float *const px = m->pr_x + (size_t)(c & 1) * cap * m->n_in, *const raw = m->pr_out + (size_t)(c & 1) * cap * E;
+            std::memcpy(hx, x + r0 * m->n_in, sizeof(float) * (size_t)B * m->n_in);
+            // alone, a chunk is copied on the stream that evaluates it
+            hipStream_t up = nc > 1 ? m->pr_stream : m->stream;
+            HIPCK(hipMemcpyAsync(px, hx, sizeof(float) * (size_t)B * m->n_in, hipMemcpyHostToDevice, up));
+            if (nc > 1) {
+                HIPCK(hipEventRecord(m->pr_up, up));
+                HIPCK(hipStreamWaitEvent(m->stream, m->pr_up, 0));
+            }
             if (fused) {
-                m->infer(m->pr_x, B, raw, B0);
+                m->infer(px, B, raw, B);
             } else {
                 const size_t n = (size_t)B * m->n_in;
-                hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, m->pr_x,
+                hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, px,
                                    (const float *)nullptr, (const int *)nullptr, B, m->n_in, m->mean, m->istd, 0.f, 1.f,
                                    m->Xl[0], (float *)nullptr);
                 HIPCK(hipGetLastError());
-                for (int e = 0; e < m->members; ++e) {
+                for (int e = 0; e < E; ++e) {
                     m->forward(e, B);
-                    HIPCK(hipMemcpyAsync(raw + (size_t)e * B0, m->Zl[m->depth], sizeof(float) * B, hipMemcpyDeviceToDevice,
+                    HIPCK(hipMemcpyAsync(raw + (size_t)e * B, m->Zl[m->depth], sizeof(float) * B, hipMemcpyDeviceToDevice,
                                          m->stream));
                 }
             }
-            hipLaunchKernelGGL(casim::k_na_reduce, dim3((B + 255) / 256), dim3(256), 0, m->stream, raw, m->members, B0, B,
-                               m->ys, m->ym, mu, sd, 1);
+            hipLaunchKernelGGL(casim::k_na_reduce, dim3((B + 255) / 256), dim3(256), 0, m->stream, (const float *)raw, E, B, B,
+                               m->ys, m->ym, ho + (size_t)E * B, ho + (size_t)(E + 1) * B, ho, B);
             HIPCK(hipGetLastError());
-            if (mean) HIPCK(hipMemcpyAsync(mean + r0, mu, sizeof(float) * B, hipMemcpyDeviceToHost, m->stream));
-            if (spread) HIPCK(hipMemcpyAsync(spread + r0, sd, sizeof(float) * B, hipMemcpyDeviceToHost, m->stream));
-            if (member_out)
-                HIPCK(hipMemcpy2DAsync(member_out + r0, sizeof(float) * rows, raw, sizeof(float) * B0, sizeof(float) * B,
-                                       m->members, hipMemcpyDeviceToHost, m->stream));
+            HIPCK(hipEventRecord(m->pr_done[c & 1], m->stream));
         }
-        HIPCK(hipStreamSynchronize(m->stream));
+        for (int c = std::max(0, nc - 2); c < nc; ++c) take(c);
     });
 }
 
@@ -1555,7 +1609,7 @@ int casim_mlp_predict_noalloc(CasimMLP *m, const float *x, int64_t rows, float *
             HIPCK(hipGetLastError());
         }
         hipLaunchKernelGGL(casim::k_na_reduce, dim3((B + 255) / 256), dim3(256), 0, st, outm, m->members, cap, B, m->ys, m->ym,
-                           mean, spread, 0);
+                           mean, spread, (float *)nullptr, 0);
         HIPCK(hipGetLastError());
     });
 }
