@@ -873,11 +873,16 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
                 "with a cytosol box, k_steps must be a multiple of its substeps");
         d->use();
         const bool flat = casim::site2d_ok(d);
-        if (flat || casim::resident_ok(d, k_steps)) {
+        if (flat || casim::resident_ok(d, d->box ? M : k_steps)) {
             for (int32_t left = k_steps; left > 0;) {
-                const int32_t kc = std::min(left, (int32_t)2048);
+                // with a box, a launch covers the steps between two of its own
+                const int32_t kc = d->box ? M : std::min(left, (int32_t)2048);
                 left -= kc;
                 flat ? casim::site2d_steps(d, dt, kc) : casim::resident_steps(d, dt, kc);
+                if (d->box) {  // box step on the accumulated effluxes, then the rim
+                    casim::box_step(d, M * dt);
+                    casim::box_rim(d);
+                }
                 // the update that the next launch's first step expects
                 if (d->Q.on && d->Q.cyto) d->launch_rim(d->Q.cions, d->Q.cbb);
                 d->launch_efflux();

@@ -394,6 +394,16 @@ void box_free(CasimDyad *d) {
     d->box = nullptr;
 }
 
+bool box_links(const CasimDyad *d, BoxLinks *out) {
+    if (out) *out = BoxLinks{};
+    if (!d->box) return true;
+    const BoxArgs &a = d->box->a;
+    if (d->P.dim != 2 || a.ne > 3) return false;
+    for (int e = 0; e < a.ne; ++e)
+        if (a.ex_grid[e] != e) return false;
+    if (out) *out = {a.ne, a.nlink, {a.ex_D[0], a.ex_D[1], a.ex_D[2]}, a.link_fac, a.acc};
+    return true;
+}
 int box_substeps(const CasimDyad *d) { return d->box ? d->box->substeps : 1; }
 int box_cur(const CasimDyad *d) { return d->box ? d->box->cur : 0; }
 void box_set_cur(CasimDyad *d, int cur) {

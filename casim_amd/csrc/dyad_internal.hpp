@@ -183,6 +183,17 @@ void box_rim(CasimDyad *d);
 void box_reset(CasimDyad *d);
 void box_free(CasimDyad *d);
 int box_substeps(const CasimDyad *d);
+// What a kernel that steps the dyad over a whole box step adds up itself: the
+// exchanged fields (grid fields 0 .. ne - 1 of a 2D dyad), their diffusion, the
+// link factors and the accumulator.  False where that does not describe the
+// box; without a box ne = 0.
+struct BoxLinks {
+    int ne, nlink;
+    double D[3];
+    const double *fac;
+    double *acc;
+};
+bool box_links(const CasimDyad *d, BoxLinks *out);
 int box_cur(const CasimDyad *d);
 void box_set_cur(CasimDyad *d, int cur);
 }  // namespace casim

@@ -72,6 +72,11 @@ struct ResArgs {
     double cq, Vjsr, Velem, nCQ, KCQ, tau;
     double *jions, *jnew, *IjSR, *jnsr;
     const double *nsr;
+    // cytosol box (2D sites): exchanged fields 0 .. ne - 1, its accumulator
+    int ne, nlink;
+    double exD[3];
+    const double *link_fac;
+    double *acc;
 };
 
 // SRPool::Update and SRPool::Run (SRPool.cpp:55-89) of one site held in
@@ -108,13 +113,16 @@ __device__ __forceinline__ T xld(const T *p) {
 __device__ __forceinline__ void stores_out() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // LDS of one workgroup.
-template <typename T, int NG, int PL, int PH, int PS>
+template <typename T, int NG, int PL, int PH, int PS, bool FLAT>
 struct ResLds {
     static constexpr int SP = PH > 2 ? PH : 2;  // planes per staging buffer
     T stage[2][SP][NG][PS];
     double pg[2][RES_CH], jv[RES_CH], jvp[2];  // state * conductance, jSR of the mouth entries; the pool's jSR
     double jn[36];                             // jump of the streams over a step (high and low 16 bits of each word)
-    unsigned char map[PL][RES_CH];             // mouth entry + 1 of each (slot, y) on z = 0, 0: none
+    unsigned char map[PL][FLAT ? PS : RES_CH];  // mouth entry + 1 of each (slot, y) on z = 0, 0: none
+    // accumulated effluxes: of the links to the y-rims per slot, half, side and
+    // field, of those to the x-rims per field and lane
+    double yacc[FLAT ? PL * 12 : 1], xacc[FLAT ? 3 * PS : 1];
     int abort;
     unsigned ready;  // steps of which the neighbours' edge planes are out
     int unit;
@@ -142,13 +150,18 @@ __device__ __forceinline__ bool wait_flags(const unsigned *watch, unsigned targe
 // ---------------------------------------------------------------------------
 // waves of a workgroup for planes of PS nodes, and per SIMD
 constexpr int res_waves(int PS) { return (PS + 63) / 64 + 1; }
-template <typename T, int PL, int PH, int PS>
+// FLAT: 2D sites with four grid fields (the coupled cleft), two slabs to a
+// workgroup: lanes 0 .. ny - 1 hold the columns y of the first, ny .. 2 ny - 1
+// those of the second, which takes the place of z.  The two pass their edge
+// rows to each other through the staging buffer of phase 0.  Lanes past the
+// nodes add up the effluxes across the y-rims from the staged rows.
+template <typename T, int PL, int PH, int PS, bool FLAT>
 __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k_resident(const T *__restrict__ gin,
                                                                             T *__restrict__ gout,
                                                                             const T *__restrict__ fin,
                                                                             T *__restrict__ fout, const Params p,
                                                                             const ResArgs r, double dt_) {
-    constexpr int NG = 3, NF = 1, LY = 1, H = PL / 2;
+    constexpr int DIM = FLAT ? 2 : 3, NG = FLAT ? 4 : 3, NF = 1, LY = FLAT ? 2 : 1, H = PL / 2;
     constexpr int NPH = 1 + (PL - 2 + PH - 1) / PH;  // phases (barriers) per step
     static_assert(NPH % 2 == 0, "the staging buffers alternate over the phases of a step");
     constexpr int EB = NPH > 2 ? 2 : 1;   // barrier before which the edge planes' stores are out
@@ -156,7 +169,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
     constexpr int RNG = NPH > 2 ? 3 : 0;  // phase in which it forms the next draws
     constexpr int DM = H - 1 < PL - 2 - H ? H - 1 : PL - 2 - H, DMAX = DM < 3 ? DM : 3;
     static_assert(H - 1 - DMAX >= (H - 1) / PH * PH + 1 - PH, "slot H - 1 - d is staged one phase before slot H at most");
-    using Lds = ResLds<T, NG, PL, PH, PS>;
+    using Lds = ResLds<T, NG, PL, PH, PS, FLAT>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     Lds &S = *reinterpret_cast<Lds *>(smem);
     T *faces = reinterpret_cast<T *>(smem + sizeof(Lds));  // [2 * ny][PLF]
@@ -182,6 +195,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
     const int np = base + (gi < extra ? 1 : 0);               // planes of this slab
     const int x0 = 1 + gi * base + min(gi, extra);            // first of them
     const int x1 = x0 + np;
+    const int npa = FLAT ? (np + 1) / 2 : np;  // of the first half
     const int d = PL - np;  // slots that repeat a plane (0 .. DMAX)
     const int P = p.ny * p.nz;
     const size_t fs = (size_t)p.S * p.NS;
@@ -202,14 +216,29 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
     if (wave < r.nw) {
         // ---- node waves ---------------------------------------------------
         const int q = threadIdx.x;
-        const bool act = q < P;
-        const int z = q % p.nz, y = q / p.nz;
+        const bool act = q < (FLAT ? 2 * P : P);
+        const int z = FLAT ? q >= P : q % p.nz, y = FLAT ? q - z * P : q / p.nz;  // FLAT: z is the half
+        const int yq = FLAT ? y : q, mi = FLAT ? q : y;  // index in a plane of the state, in the mouth map
+        const bool mouths = FLAT ? act : z == 0 && act;
         const bool inner = act && y >= 1 && y <= p.ny - 2;
         const int zl = z == 0 ? 1 : -1, zr = z == p.nz - 1 ? -1 : 1;
-        const bool face = act && (z == 0 || z == p.nz - 1);
+        const bool face = !FLAT && act && (z == 0 || z == p.nz - 1);
         T *const fl = faces + ((z == 0 ? 0 : p.ny) + (act ? y : 0)) * PLF;  // this node's face values, one per slot
         const int fg = (z == 0 ? 0 : p.nFP) + (act ? y : 0);
         const T ihx2 = (T)p.ihx2, ihy2 = (T)p.ihy2, ihz2 = (T)p.ihz2;
+        // this lane's slab: its first plane, the plane after its last, its doubled slots
+        const int lx0 = FLAT && z ? x0 + npa : x0, lx1 = FLAT && !z ? x0 + npa : x1, ld = FLAT ? PL - (lx1 - lx0) : d;
+        // effluxes across the y-rims: lane al takes half al & 1, side al >> 1 & 1 and
+        // field (al >> 2) % 3 of every third plane of a phase
+        const int al = FLAT && r.ne ? q - 2 * P : -1, asub = al / 12, af = al < 0 ? 0 : (al >> 2) % 3;
+        const bool acc_lane = FLAT && al >= 0 && al < 36 && af < r.ne;
+        const int arim = (al & 1) * P + (al >> 1 & 1 ? P - 1 : 0), ain = arim + (al >> 1 & 1 ? -1 : 1);
+        const double exd = FLAT ? (af == 0 ? r.exD[0] : af == 1 ? r.exD[1] : r.exD[2]) : 0.0;
+        const double facx = FLAT && r.ne ? r.link_fac[0] : 0.0, facy = FLAT && r.ne ? r.link_fac[2 * (P - 2)] : 0.0;
+        auto flux = [&](double v, double D, double fac, double u, double ur) {  // k_box_efflux
+#pragma clang fp contract(off)
+            return v + dt_ * (D * (fac * (u - ur)));
+        };
         for (int s = grp; s < p.S; s += r.groups) {
             __syncthreads();  // the last site's tables are free
             if (aborted()) return;
@@ -219,8 +248,9 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
             {
                 // opaque copies: the planes' offsets are formed here and at the
                 // write-out, not kept in registers over the steps and sites
-                int lo = x0, hi = x1 - PL, qo = q, fo = fg;
-                asm volatile("" : "+s"(lo), "+s"(hi), "+v"(qo), "+v"(fo));
+                int lo = lx0, hi = lx1 - PL, qo = yq, fo = fg;
+                if constexpr (FLAT) asm volatile("" : "+v"(lo), "+v"(hi), "+v"(qo));
+                else asm volatile("" : "+s"(lo), "+s"(hi), "+v"(qo), "+v"(fo));
 #pragma unroll
                 for (int i = 0; i < PL; ++i) {
                     const int x = i + (i < H ? lo : hi);
@@ -228,7 +258,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                     for (int g = 0; g < NG; ++g)
                         R[i][g] = act ? ld_off(gs + g * fs, (unsigned)((x * P + qo) * (int)sizeof(T))) : (T)0;
                     if (face) fl[i] = ffs[fo + x * p.ny];
-                    if (z == 0 && act) S.map[i][y] = 0;
+                    if (mouths) S.map[i][mi] = 0;
                 }
             }
             // planes next to the slab: the rim planes, or the neighbours' edge
@@ -236,22 +266,27 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
             T hl[NG], hr[NG];
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
-                hl[g] = act ? ld_off(gs + g * fs, (unsigned)(((x0 - 1) * P + q) * (int)sizeof(T))) : (T)0;
-                hr[g] = act ? ld_off(gs + g * fs, (unsigned)((x1 * P + q) * (int)sizeof(T))) : (T)0;
+                hl[g] = act ? ld_off(gs + g * fs, (unsigned)(((lx0 - 1) * P + yq) * (int)sizeof(T))) : (T)0;
+                hr[g] = act ? ld_off(gs + g * fs, (unsigned)((lx1 * P + yq) * (int)sizeof(T))) : (T)0;
+            }
+            if (FLAT && r.ne) {
+                for (int i = q; i < PL * 12; i += r.nw * 64) S.yacc[i] = 0.0;
+                for (int e = 0; e < 3; ++e)
+                    if (q < PS) S.xacc[e * PS + q] = 0.0;
             }
             __syncthreads();  // map cleared: the channel wave enters the mouths
             __syncthreads();
             using Mask = std::conditional_t<(PL > 32), uint64_t, uint32_t>;
             Mask mask = 0;  // slots in which this node is a mouth
-            if (z == 0 && act)
+            if (mouths)
 #pragma unroll
                 for (int i = 0; i < PL; ++i)
-                    if (S.map[i][y]) mask |= (Mask)1 << i;
+                    if (S.map[i][mi]) mask |= (Mask)1 << i;
             if (mask) {
                 double *mo = mouth_at(E);
 #pragma unroll
                 for (int i = 0; i < PL; ++i)
-                    if (mask >> i & 1) xst(mo + S.map[i][y] - 1, (double)R[i][0]);
+                    if (mask >> i & 1) xst(mo + S.map[i][mi] - 1, (double)R[i][0]);
             }
 
             T prev[NG], last[NG];
@@ -275,8 +310,8 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                     const int o = (i * NG + g) * PS;
                     n.v[0][g] = b.yl[o];
                     n.v[1][g] = b.yr[o];
-                    n.v[2][g] = b.zl[o];
-                    n.v[3][g] = b.zr[o];
+                    if (!FLAT) n.v[2][g] = b.zl[o];
+                    if (!FLAT) n.v[3][g] = b.zr[o];
                 }
                 // doubles issued here: left to itself the scheduler puts each pair of reads
                 // next to its sum and waits for every pair in turn (4096 sites of 81x81x5:
@@ -289,15 +324,16 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                 const T Fv[NF] = {F};
                 const T J[1] = {J0};
                 T Fo[NF] = {F};
-                node_update<T, 3, 1, 3, NG, NF, LY>(p, Cm, R[i], Cp, nb, z, face, Fv, J, dt, ihx2, ihy2, ihz2, O, Fo);
+                node_update<T, DIM, 1, 3, NG, NF, LY>(p, Cm, R[i], Cp, nb, z, face, Fv, J, dt, ihx2, ihy2, ihz2, O, Fo);
                 F = Fo[0];
                 // one plane at a time: without this the compiler gathers every
                 // plane's neighbours at the head of a phase and spills
-                asm volatile("" : "+v"(O[0]), "+v"(O[1]), "+v"(O[2])::"memory");
+                if constexpr (FLAT) asm volatile("" : "+v"(O[0]), "+v"(O[1]), "+v"(O[2]), "+v"(O[NG - 1])::"memory");
+                else asm volatile("" : "+v"(O[0]), "+v"(O[1]), "+v"(O[2])::"memory");
             };
             // the current of a mouth node: state * conductance as gated, times jSR - mouth
             auto current = [&](int i, int par) {
-                const int e = S.map[i][y] - 1;
+                const int e = S.map[i][mi] - 1;
                 const double jvv = pool ? S.jvp[par] : S.jv[e];
                 return (T)(S.pg[par][e] * (jvv - (double)R[i][0]));
             };
@@ -318,15 +354,27 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                 return (int)(__builtin_amdgcn_readfirstlane(*(volatile unsigned *)&S.ready) - t) >= 0;
             };
             auto halos = [&](int k1) {
-                if (act && gi > 0) {
+                if (act && gi > 0 && !(FLAT && z)) {
                     const T *e = edge_at(unit - 1, E + k1, 1);
 #pragma unroll
-                    for (int g = 0; g < NG; ++g) hl[g] = xld(e + g * PS + q);
+                    for (int g = 0; g < NG; ++g) hl[g] = xld(e + g * PS + yq);
                 }
-                if (act && gi < r.G - 1) {
+                if (act && gi < r.G - 1 && !(FLAT && !z)) {
                     const T *e = edge_at(unit + 1, E + k1, 0);
 #pragma unroll
-                    for (int g = 0; g < NG; ++g) hr[g] = xld(e + g * PS + q);
+                    for (int g = 0; g < NG; ++g) hr[g] = xld(e + g * PS + yq);
+                }
+            };
+            // the y-rims' effluxes of the planes staged for phase j
+            auto effluxes = [&](int j) {
+                const int i0 = 1 + (j - 1) * PH, i1 = i0 + PH < PL - 1 ? i0 + PH : PL - 1;
+                const T *c = &S.stage[j & 1][0][af][0];
+#pragma unroll
+                for (int i = 0; i < PH; ++i) {
+                    const int l = j ? i0 + i : i ? PL - 1 : 0;
+                    if (!(j ? l < i1 : i < 2) || i % 3 != asub) continue;
+                    double &v = S.yacc[l * 12 + al % 12];
+                    v = flux(v, exd, facy, (double)c[i * NG * PS + ain], (double)c[i * NG * PS + arim]);
                 }
             };
             stage(0);
@@ -349,6 +397,19 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                     prev[g] = R[0][g];
                     last[g] = R[PL - 1][g];
                 }
+                if (FLAT && acc_lane) effluxes(0);
+                if (FLAT && r.ne && inner) {
+                    // across the x-rims
+                    if (gi == 0 && !z)
+#pragma unroll
+                        for (int e = 0; e < 3; ++e)
+                            if (e < r.ne) S.xacc[e * PS + q] = flux(S.xacc[e * PS + q], r.exD[e], facx, (double)R[0][e], (double)hl[e]);
+                    if (gi == r.G - 1 && z)
+#pragma unroll
+                        for (int e = 0; e < 3; ++e)
+                            if (e < r.ne)
+                                S.xacc[e * PS + q] = flux(S.xacc[e * PS + q], r.exD[e], facx, (double)R[PL - 1][e], (double)hr[e]);
+                }
                 if (inner) {
                     T J0 = (T)0, J1 = (T)0;
                     const bool hot = (mask & ((Mask)1 | (Mask)1 << (PL - 1))) != 0;
@@ -363,8 +424,22 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                     }
                     const Beside bs = beside(column(0));
                     const Nbr b0 = nbrs(bs, 0), b1 = nbrs(bs, 1);
-                    update(0, b0, hl, R[1], F0, J0, n0);
-                    update(PL - 1, b1, R[PL - 2], hr, F1, J1, n1);
+                    if constexpr (FLAT) {
+                        // the halves' inner edges: the second's first row, the first's last one
+                        const LdsT *o = column(0) + (z ? NG * PS - P : P);
+                        T ml[NG], mr[NG];
+#pragma unroll
+                        for (int g = 0; g < NG; ++g) {
+                            const T v = o[g * PS];
+                            ml[g] = z ? v : hl[g];
+                            mr[g] = z ? hr[g] : v;
+                        }
+                        update(0, b0, ml, R[1], F0, J0, n0);
+                        update(PL - 1, b1, R[PL - 2], mr, F1, J1, n1);
+                    } else {
+                        update(0, b0, hl, R[1], F0, J0, n0);
+                        update(PL - 1, b1, R[PL - 2], hr, F1, J1, n1);
+                    }
                     if (face) {
                         fl[0] = F0;
                         fl[PL - 1] = F1;
@@ -375,16 +450,22 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                         R[PL - 1][g] = n1[g];
                     }
                     if (r.G > 1 && k + 1 < r.K) {
-                        T *e0 = edge_at(unit, E + k + 1, 0) + q, *e1 = edge_at(unit, E + k + 1, 1) + q;
+                        if constexpr (FLAT) {
+                            T *e = edge_at(unit, E + k + 1, z) + y;
 #pragma unroll
-                        for (int g = 0; g < NG; ++g) {
-                            xst(e0 + g * PS, R[0][g]);
-                            xst(e1 + g * PS, R[PL - 1][g]);
+                            for (int g = 0; g < NG; ++g) xst(e + g * PS, z ? R[PL - 1][g] : R[0][g]);
+                        } else {
+                            T *e0 = edge_at(unit, E + k + 1, 0) + q, *e1 = edge_at(unit, E + k + 1, 1) + q;
+#pragma unroll
+                            for (int g = 0; g < NG; ++g) {
+                                xst(e0 + g * PS, R[0][g]);
+                                xst(e1 + g * PS, R[PL - 1][g]);
+                            }
                         }
                     }
                     if (hot && k + 1 < r.K) {
-                        if (mask & 1u) xst(mo + S.map[0][y] - 1, (double)R[0][0]);
-                        if (mask >> (PL - 1) & 1u) xst(mo + S.map[PL - 1][y] - 1, (double)R[PL - 1][0]);
+                        if (mask & 1u) xst(mo + S.map[0][mi] - 1, (double)R[0][0]);
+                        if (mask >> (PL - 1) & 1u) xst(mo + S.map[PL - 1][mi] - 1, (double)R[PL - 1][0]);
                     }
                 }
                 // the planes between them
@@ -396,8 +477,8 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                     // with d > 0 the lower neighbour of slot H is slot H - 1 - d, whose old
                     // values this thread has staged for this phase or the one before
                     T keep[NG];
-                    if (H >= i0 && H < i1 && d) {
-                        const int l = H - 1 - d;
+                    if (H >= i0 && H < i1 && (FLAT ? act : d != 0)) {
+                        const int l = H - 1 - ld;  // FLAT: the halves may differ, and with ld == 0 it is prev
                         LdsT *lp = l >= i0 ? column(j & 1) + (l - i0) * NG * PS
                                            : column((j & 1) ^ 1) + (l == 0 ? 0 : l - (i0 - PH)) * NG * PS;
 #pragma unroll
@@ -409,6 +490,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                     }
                     // the next phase's planes go out while this one is computed
                     if (j + 1 < NPH || k + 1 < r.K) stage(j + 1 < NPH ? j + 1 : 0);
+                    if (FLAT && acc_lane) effluxes(j);
                     if (inner) {
                         T J[PH], F[PH];
 #pragma unroll
@@ -431,14 +513,14 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                             T lo[NG], hi[NG], n[NG];
 #pragma unroll
                             for (int g = 0; g < NG; ++g) {
-                                lo[g] = i == H && d ? keep[g] : prev[g];
+                                lo[g] = i == H && (FLAT || d) ? keep[g] : prev[g];
                                 hi[g] = i + 1 == PL - 1 ? last[g] : R[i + 1][g];
                             }
                             if (i == H - 1) {
 #pragma unroll
                                 for (int e = 1; e <= DMAX; ++e)
 #pragma unroll
-                                    for (int g = 0; g < NG; ++g) hi[g] = d == e ? R[H + e][g] : hi[g];
+                                    for (int g = 0; g < NG; ++g) hi[g] = ld == e ? R[H + e][g] : hi[g];
                             }
                             update(i, nb, lo, hi, F[i - i0], J[i - i0], n);
 #pragma unroll
@@ -454,19 +536,34 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                         if (hot && k + 1 < r.K)
 #pragma unroll
                             for (int i = i0; i < i1; ++i)
-                                if (mask >> i & 1u) xst(mo + S.map[i][y] - 1, (double)R[i][0]);
+                                if (mask >> i & 1u) xst(mo + S.map[i][mi] - 1, (double)R[i][0]);
                     }
                 }
             }
             // the slab's planes, rim nodes included (each plane in one slot)
             T *os = gout + (size_t)s * p.NS;
             T *ofs = fout + (size_t)s * 2 * p.nFP;
+            if (FLAT && acc_lane) {
+                const int h0 = al & 1 ? x0 + npa : x0, h1 = al & 1 ? x1 : x0 + npa, hd = PL - (h1 - h0);
+                double *to = r.acc + ((size_t)af * p.S + s) * r.nlink + 2 * (P - 2) + (al >> 1 & 1) * N;
+#pragma unroll 1
+                for (int i = 0; i < PL; ++i) {
+                    const int at = i == 0 ? 0 : i == PL - 1 ? 1 : (i - 1) % PH;  // its place in its phase
+                    if (at % 3 != asub || (i >= H && i < H + hd)) continue;
+                    to[(i < H ? h0 + i : h1 - PL + i) - 1] = S.yacc[i * 12 + al % 12];
+                }
+            }
+            if (FLAT && r.ne && inner && (z ? gi == r.G - 1 : gi == 0))
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (e < r.ne) r.acc[((size_t)e * p.S + s) * r.nlink + z * (P - 2) + y - 1] = S.xacc[e * PS + q];
             if (act) {
-                int lo = x0, hi = x1 - PL, qo = q, fo = fg;
-                asm volatile("" : "+s"(lo), "+s"(hi), "+v"(qo), "+v"(fo));
+                int lo = lx0, hi = lx1 - PL, qo = yq, fo = fg;
+                if constexpr (FLAT) asm volatile("" : "+v"(lo), "+v"(hi), "+v"(qo));
+                else asm volatile("" : "+s"(lo), "+s"(hi), "+v"(qo), "+v"(fo));
 #pragma unroll
                 for (int i = 0; i < PL; ++i) {
-                    if (i >= H && i < H + d) continue;
+                    if (i >= H && i < H + ld) continue;
                     const int x = i + (i < H ? lo : hi);
 #pragma unroll
                     for (int g = 0; g < NG; ++g) st_off(os + g * fs, (unsigned)((x * P + qo) * (int)sizeof(T)), R[i][g]);
@@ -538,9 +635,10 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
         for (int e = elo + lane; e < ehi; e += 64) {
             if (e + 1 < n && sn[e + 1] == sn[e]) continue;  // the last channel on a node wins
             const int x = sn[e] / P, yy = (sn[e] - x * P) / p.nz;
-            const int lo = x - x0, hi = x - x1 + PL;  // its slots
-            if (lo < H) S.map[lo][yy] = (unsigned char)(e + 1);
-            if (hi >= H) S.map[hi][yy] = (unsigned char)(e + 1);
+            const int half = FLAT && x >= x0 + npa, h0 = half ? x0 + npa : x0, h1 = FLAT && !half ? x0 + npa : x1;
+            const int lo = x - h0, hi = x - h1 + PL, at = half ? P + yy : yy;  // its slots
+            if (lo < H) S.map[lo][at] = (unsigned char)(e + 1);
+            if (hi >= H) S.map[hi][at] = (unsigned char)(e + 1);
         }
         // stream: per channel the state one step into its draw if no channel
         // toggles before it in the step, and the draw's first value
@@ -780,24 +878,25 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
 constexpr int RES_CUS = 256;  // CUs, one workgroup each (registers and LDS of a CU)
 
 struct Form {
-    int PL, PH, PS;
+    int PL, PH, PS, flat;
     int f64;
     double us0, us1;  // measured: a step of the sites on the chip takes us0 + us1 * PL
     size_t lds;
     void (*launch)(CasimDyad *, double, const ResArgs &, size_t);
 };
 
-template <typename T, int PL, int PH, int PS>
+template <typename T, int PL, int PH, int PS, bool FLAT>
 void launch_form(CasimDyad *d, double dt, const ResArgs &r, size_t lds) {
-    auto *k = k_resident<T, PL, PH, PS>;
+    auto *k = k_resident<T, PL, PH, PS, FLAT>;
     HIPCK(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, dim3(r.units), dim3((r.nw + 1) * 64), lds, d->stream, (const T *)d->g[d->cur],
                        (T *)d->g[d->cur ^ 1], (const T *)d->f[d->cur], (T *)d->f[d->cur ^ 1], d->P, r, dt);
     HIPCK(hipGetLastError());
 }
-template <typename T, int PL, int PH, int PS>
+template <typename T, int PL, int PH, int PS, bool FLAT = false>
 Form form(double us0, double us1) {
-    return {PL, PH, PS, sizeof(T) == 8, us0, us1, sizeof(ResLds<T, 3, PL, PH, PS>), launch_form<T, PL, PH, PS>};
+    return {PL,  PH,  PS, FLAT, sizeof(T) == 8, us0, us1, sizeof(ResLds<T, FLAT ? 4 : 3, PL, PH, PS, FLAT>),
+            launch_form<T, PL, PH, PS, FLAT>};
 }
 const Form FORMS[] = {
     form<double, 20, 4, 440>(2.1, 0.37), form<double, 10, 3, 440>(2.1, 0.37), form<double, 5, 3, 440>(2.1, 0.37),
@@ -807,6 +906,9 @@ const Form FORMS[] = {
     // 200 sites 17.5 -> 7.1, FP32 2500 sites 41.6 -> 30.7; FP64 2500 sites 73.5, 79.8 here, so by the sweeps)
     form<double, 10, 3, 576>(0.6, 0.94), form<double, 5, 3, 576>(0.6, 0.94), form<float, 20, 6, 576>(3.7, 0.18),
     form<float, 10, 3, 576>(3.7, 0.18),  form<float, 5, 3, 576>(3.7, 0.18),
+    // two slabs of 2D columns to a workgroup (201x201, 100 steps, ms, the sweeps before: 1 site 10.8 -> 0.53,
+    // 200 sites 15.0 -> 4.0, 800 sites 24.0 -> 15.8, FP32 800 sites 16.5 -> 8.7; 20 planes of doubles would spill)
+    form<double, 17, 3, 412, true>(1.0, 0.39), form<double, 10, 3, 412, true>(1.0, 0.39), form<float, 20, 6, 412, true>(2.0, 0.17),
 };
 
 }  // namespace
@@ -832,20 +934,25 @@ bool resident_ok(CasimDyad *d, int K) {
         const double here = rounds * (25.0 + 0.5 * f.PL + K * (f.us0 + f.us1 * f.PL));
         return here <= K * (40.0 + (f.f64 ? 5.9e-6 : 3.3e-6) * (double)p.S * (double)p.NS);
     };
-    if (!d->chan_small || d->box || (d->Q.on && d->Q.cyto) || d->steps_per_pass < 2 || !d->use_sweep) return false;
-    if (p.dim != 3 || layout_id(p) != 1 || p.nz < 2 || p.ny > RES_CH || d->M >= RES_CH) return false;
+    const bool flat = p.dim == 2;
+    if (!d->chan_small || (d->Q.on && d->Q.cyto) || d->steps_per_pass < 2 || !d->use_sweep || d->M >= RES_CH) return false;
+    if (flat ? layout_id(p) != 2 || !box_links(d, nullptr) : d->box || layout_id(p) != 1 || p.nz < 2 || p.ny > RES_CH)
+        return false;
     if (d->res_tried) return d->res != nullptr && pays();
     d->res_tried = true;
     const int N = p.nx - 2, P = p.ny * p.nz;
+    auto lds_of = [&](const Form &f) { return f.lds + (flat ? 0 : (size_t)(f.PL | 1) * 2 * p.ny * d->tsize); };
     const Form *best = nullptr;
     int bg = 0;
     double cost = 1e300;
     for (const Form &f : FORMS) {
-        if (f.f64 != (d->precision == CASIM_FP64) || P > f.PS) continue;
+        if (f.flat != flat || f.f64 != (d->precision == CASIM_FP64) || (flat ? 2 * P + 36 > 448 : P > f.PS)) continue;
         const int H = f.PL / 2, dmax = std::min(3, std::min(H - 1, f.PL - 2 - H));
-        if (f.lds + (size_t)(f.PL | 1) * 2 * p.ny * d->tsize > 160 * 1024) continue;
+        if (lds_of(f) > 160 * 1024) continue;
         for (int G = 1; G <= 16; ++G) {
-            const int hi = (N + G - 1) / G, lo = N / G;
+            // planes of the fullest and the emptiest slab
+            int hi = (N + G - 1) / G, lo = N / G;
+            if (flat) hi = (hi + 1) / 2, lo = lo / 2;
             if (hi > f.PL || f.PL - lo > dmax || lo < H + 1) continue;
             const int groups = std::min(p.S, RES_CUS / G);
             const double c = (p.S + groups - 1) / groups * (f.us0 + f.us1 * f.PL);
@@ -856,17 +963,17 @@ bool resident_ok(CasimDyad *d, int K) {
     auto *res = new Resident();
     d->res = res;
     res->f = best;
-    res->lds = best->lds + (size_t)(best->PL | 1) * 2 * p.ny * d->tsize;
+    res->lds = lds_of(*best);
     ResArgs &a = res->a;
     a.G = bg;
     a.groups = std::min(p.S, RES_CUS / bg);
     a.units = a.groups * bg;
-    a.nw = (P + 63) / 64;
+    a.nw = ((flat ? 2 * P + 36 : P) + 63) / 64;
     const size_t flags = (size_t)a.units * 32 * sizeof(unsigned);
     HIPCK(hipMalloc(&a.mflag, flags));
     HIPCK(hipMalloc(&a.eflag, flags));
     HIPCK(hipMalloc(&a.ticket, sizeof(*a.ticket)));
-    HIPCK(hipMalloc(&a.edge, (size_t)a.units * RES_PAR * 2 * 3 * best->PS * d->tsize));
+    HIPCK(hipMalloc(&a.edge, (size_t)a.units * RES_PAR * 2 * (flat ? 4 : 3) * best->PS * d->tsize));
     HIPCK(hipMalloc(&a.mouth, (size_t)a.groups * RES_PAR * RES_CH * sizeof(double)));
     HIPCK(hipHostMalloc((void **)&a.err, sizeof(int), hipHostMallocMapped));
     *a.err = 0;
@@ -896,6 +1003,10 @@ void resident_steps(CasimDyad *d, double dt, int k) {
     a.pool = q.on, a.jsr_const = q.jsr_const;
     a.cq = q.cq, a.Vjsr = q.Vjsr, a.Velem = q.Velem, a.nCQ = q.nCQ[0], a.KCQ = q.KCQ[0], a.tau = q.tau[0];
     a.jions = q.jions, a.jnew = q.jnew, a.IjSR = q.IjSR, a.jnsr = q.jnsr, a.nsr = q.nsr;
+    BoxLinks b{};
+    if (d->box) (void)box_links(d, &b);
+    a.ne = b.ne, a.nlink = b.nlink, a.link_fac = b.fac, a.acc = b.acc;
+    for (int e = 0; e < 3; ++e) a.exD[e] = b.D[e];
     d->res->f->launch(d, dt, a, d->res->lds);
     d->cur ^= 1;
 }

@@ -237,9 +237,10 @@ int casim_dyad_run_mc(CasimDyad *d, double dt, int32_t site);
  * graph per (step count, dt) and replayed; one graph holds at most 2048 steps
  * (with a cytosol box, the most whole box steps below that), so a longer call
  * replays several graphs, with the results of one call.  3D one-ion layouts
- * without a cytosol pool or box keep the state on the chip over the steps of a
- * call instead, where the number of steps pays for it; results do not depend
- * on that either.  casim_dyad_set_steps_per_pass(d, 1) selects the sweeps.
+ * without a cytosol pool or box, and 2D sites of the known layouts, keep the
+ * state on the chip over the steps of a call (between two box steps) instead,
+ * where the number of steps pays for it; results do not depend on that either.
+ * casim_dyad_set_steps_per_pass(d, 1) selects the sweeps.
  */
 int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps);
 

@@ -85,3 +85,36 @@ def test_equals_one_step_per_pass(gpu, kind, sites, nx, ny, precision):
     for d in (a, b):
         d.Step(dt, 41)
     same(state(a, sp, pools), state(b, sp, pools))
+
+
+# grids that take several workgroups per site, with and without a cytosol box:
+# halves of a slab that differ and that do not, rows of one wave and of three,
+# doubled rows, more sites than fit at once; the last one takes the sweeps
+@pytest.mark.parametrize("sites,nx,ny,precision,box", [
+    (3, 61, 61, 64, True), (45, 201, 201, 64, True), (2, 63, 101, 64, False), (9, 41, 61, 32, True), (4, 72, 206, 32, False),
+    (2, 68, 50, 64, True), (2, 60, 207, 64, False)])
+def test_wide_grid_equals_one_step_per_pass(gpu, sites, nx, ny, precision, box):
+    sp = workloads.coupled_dyads(sites, n_ryr=16, extent_nm=2.0 * (min(nx, ny) - 1),
+                                 precision=abi.CASIM_FP32 if precision == 32 else abi.CASIM_FP64)
+    sp.channel_types[0].params["kopen0"] *= 1e5
+    sp.channel_types[0].params["kclose0"] *= 1e4
+    c = min(nx, ny) // 2
+    sp.sites = [[(2.0 * (nx // 2 + i * (c // 4)), 2.0 * (ny // 2 + k * (c // 4)), 0) for i in range(-2, 3) for k in range(-2, 3)]
+                for _ in range(sites)]
+    sp = dataclasses.replace(sp, nx=nx, ny=ny, init_channel=[s % 25 for s in range(sites)])
+    devs = []
+    for steps_per_pass in (2, 1):
+        d = DyadHIP(sp)
+        d.AttachPools(POOL)
+        if box:
+            d.AttachCytosolBox(workloads.coupled_box(sp))
+        d.SetStepsPerPass(steps_per_pass)
+        d.RecordOpenCounts(5, 40)
+        d.InitOpeningAll()
+        d.UpdatePools(*(() if box else sp.rim_arrays()))
+        for k in (50, 150):
+            d.Step(sp.meta["dt_ms"], k)
+        out = state(d, sp, None) + [d.GetPools()[0]]
+        devs.append(out + [d.GetCytosolBox(f) for f in range(4)] if box else out)
+    same(*devs)
+    assert np.isfinite(devs[0][0]).all() and (devs[0][0] != devs[0][0].flat[0]).any()
