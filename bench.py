@@ -23,6 +23,7 @@ sys.path.insert(0, ROOT)
 
 METRIC = "simulated dyad-ms/s on 1 GPU (plain vs surrogate) at ≤2% Ca err; HBM GB/s"
 HBM_PEAK_GBS = 8000.0
+FP64_PEAK_TFLOPS = 78.6  # vector FP64, nominal
 COPY_GBS = 5314.0  # a plain 1 GiB device-to-device copy on MI355X (read + write), measured with rocprofv3 (kernel trace)
 
 
@@ -69,7 +70,10 @@ def run_gpu_leg(workloads, DyadHIP, precision, n_sites, steps, warmup, chunk, re
         dev.Step(dt, rem)
     dev.Synchronize()
     t = time.perf_counter() - t0
-    # per-kernel durations, live, with HIP events on the handle's stream
+    # durations of the sweep kernels (what steps of few, and of other layouts,
+    # take), live, with HIP events on the handle's stream, after a call that
+    # loads their code
+    dev.StepProfiled(dt, 2)
     ms_sweep, ms_chan = dev.StepProfiled(dt, steps)
     per_pass = dev.StepsPerPass()
     launches = steps // per_pass + steps % per_pass
@@ -230,6 +234,7 @@ def coupled_leg(workloads, DyadHIP, n_sites, steps, warmup, chunk=100, tuning=No
         dev.Step(dt, chunk)
     dev.Synchronize()
     t = time.perf_counter() - t0
+    dev.StepProfiled(dt, box.substeps)
     ms_sweep, ms_chan = dev.StepProfiled(dt, chunk)
     jsr = dev.GetPools()[0]
     ca = dev.GetCytosolBox(0)
@@ -325,7 +330,16 @@ def main():
         log("cpu baseline")
         cpu = cpu_baseline(workloads)
         log("cpu:", json.dumps(cpu))
-    # dominant kernel: k_sweep2 (two steps per launch) or k_sweep (one).  Its
+    # dominant kernel: k_resident, the state in registers over a call's steps;
+    # bound by FP64 issue and the barriers of a step, so priced in operations:
+    # per interior node 14 for each of the three diffusing fields and 9 for each
+    # bound field (the third on the two z-faces only).  With one step per pass
+    # the sweep takes its place.
+    resident = a.steps_per_pass == 2
+    nx, ny, nz = (int(v) for v in r64["grid"].split("x"))
+    flops = (nx - 2) * (ny - 2) * (nz * (3 * 14 + 2 * 9) + 2 * 9)
+    tflops = a.sites * flops / (r64["ms_per_step"] * 1e-3) / 1e12
+    # sweep kernels: k_sweep2 (two steps per launch) or k_sweep (one).  Their
     # algorithmic bytes per launch are one read and one write of every
     # site's state (sites x bytes per site-step): a two-step launch moves the
     # state once, so the steps it advances do not multiply the bytes.
@@ -333,6 +347,16 @@ def main():
     launch_bytes = a.sites * r64["bytes_per_site_step"]
     achieved = launch_bytes / (r64["sweep_launch_ms"] * 1e-3) / 1e9
     traffic = traffic_from_profiles(kernel)
+    sweep = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
+             "kernel": kernel, "steps_per_launch": r64["steps_per_launch"],
+             "launch_ms": r64["sweep_launch_ms"], "algorithmic_bytes_per_launch": launch_bytes,
+             # what HBM actually moves per launch (traffic / launch time), next to the copy rate
+             "physical_gbs": None if traffic is None else traffic / (r64["sweep_launch_ms"] * 1e-3) / 1e9,
+             "copy_gbs": COPY_GBS,
+             # per-step algorithmic rate: the bytes a one-step-per-pass sweep would move
+             # for the same steps, over the same time (not bounded by the HBM peak)
+             "effective_gbs": r64["steps_per_launch"] * achieved}
     out = {
         "metric": METRIC,
         "value": r64["dyad_ms_per_s"],
@@ -347,19 +371,13 @@ def main():
         "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": r64["workload"], "sites": a.sites, "grid": r64["grid"], "dt_ns": 10,
-                   "path": "plain batched RD, graph of %d steps%s" % (
-                       min(a.chunk, a.steps), "" if a.no_split else ", two half-batch streams"),
+                   "path": "plain batched RD, calls of %d steps%s" % (
+                       min(a.chunk, a.steps), ", state on the chip" if resident else ", one step per pass"),
                    "tuning": r64["tuning"]},
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": kernel, "steps_per_launch": r64["steps_per_launch"],
-                     "launch_ms": r64["sweep_launch_ms"], "algorithmic_bytes_per_launch": launch_bytes,
-                     # what HBM actually moves per launch (traffic / launch time), next to the copy rate
-                     "physical_gbs": None if traffic is None else traffic / (r64["sweep_launch_ms"] * 1e-3) / 1e9,
-                     "copy_gbs": COPY_GBS,
-                     # per-step algorithmic rate: the bytes a one-step-per-pass sweep would move
-                     # for the same steps, over the same time (not bounded by the HBM peak)
-                     "effective_gbs": r64["steps_per_launch"] * achieved},
+        "roofline": {"bound": "fp64", "achieved": tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": tflops / FP64_PEAK_TFLOPS, "kernel": "k_resident",
+                     "flops_per_site_step": flops} if resident else sweep,
+        "sweep": sweep,
         "cpu_baseline": cpu,
         # one-step-per-pass bytes of a whole step (channels + sweep) over its time
         "effective_gbs_whole_step": a.sites * r64["bytes_per_site_step"] / (r64["ms_per_step"] * 1e-3) / 1e9,
