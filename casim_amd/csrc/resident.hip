@@ -20,16 +20,17 @@
 // earlier sites end.
 //
 // What bounds it: the row of barriers.  At 20 planes of doubles a step takes
-// 9.4 us on every CU, of which FP64 issue of the fullest SIMD is 4 us; without
-// the arithmetic the barriers and the channel wave alone take 6.4 us.  Fewer
+// 9.0 us on every CU, of which FP64 issue of the fullest SIMD is 5 us; with
+// phases of four planes (9.4 us) the barriers and the channel wave alone took
+// 6.4 us.  In FP32 40 planes take 12 us, 10 us of them issue.  Fewer
 // planes per slab finish a step sooner, more planes carry more sites at once.
 // Measured (81x81x5, us per step; k_sweep2 with the channel kernels before):
 //   sites   FP64 k_sweep2   FP64 here   FP32 k_sweep2   FP32 here
 //       1        98             4.2           -             -
 //       6        99             4.3           -             3.7
 //      32       106             6.8           -             -
-//    1024         -           153             -            98
-//    4096       780           609           440           394
+//    1024         -           144             -            98
+//    4096       780           572           440           392
 // More workgroups per CU (128 registers each) took 765 and 362; two planes at a
 // time 604; waves waiting for their neighbour waves by LDS counters in place of
 // barriers 919 and more.
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                 }
                 // doubles issued here: left to itself the scheduler puts each pair of reads
                 // next to its sum and waits for every pair in turn (4096 sites of 81x81x5:
-                // 0.61 ms per step, 0.71 without; FP32 0.40, 0.39 without)
+                // 0.61 ms per step, 0.71 without, with phases of four planes; FP32 0.40, 0.39 without)
                 if (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
                 return n;
             };
@@ -899,7 +900,9 @@ Form form(double us0, double us1) {
             launch_form<T, PL, PH, PS, FLAT>};
 }
 const Form FORMS[] = {
-    form<double, 20, 4, 440>(2.1, 0.37), form<double, 10, 3, 440>(2.1, 0.37), form<double, 5, 3, 440>(2.1, 0.37),
+    // fewer phases as LDS allows: six planes each fit up to 408 nodes (4096 sites: 572 us per step, 599 with four)
+    form<double, 20, 6, 408>(2.1, 0.343), form<double, 20, 4, 440>(2.1, 0.37), form<double, 10, 3, 440>(2.1, 0.37),
+    form<double, 5, 3, 440>(2.1, 0.37),
     form<float, 40, 8, 440>(2.0, 0.25),  form<float, 20, 6, 440>(2.0, 0.25),  form<float, 10, 3, 440>(2.0, 0.25),
     form<float, 5, 3, 440>(2.0, 0.25),
     // three waves per SIMD, 168 registers (81x96x6, 100 steps, ms, the sweeps before: 32 sites 15.2 -> 1.1,

@@ -63,7 +63,7 @@ def same(a, b):
 # fit and take the sweeps
 @pytest.mark.parametrize("sites,nx,ny,nz,precision,pool", [
     (1, 81, 81, 5, 64, False), (7, 48, 88, 5, 64, True), (3, 59, 61, 2, 64, False), (40, 81, 79, 5, 64, False),
-    (90, 73, 64, 4, 64, True), (30, 52, 52, 5, 64, False), (2, 95, 77, 5, 32, True), (150, 81, 81, 5, 32, False),
+    (40, 81, 88, 5, 64, True), (90, 73, 64, 4, 64, True), (30, 52, 52, 5, 64, False), (2, 95, 77, 5, 32, True), (150, 81, 81, 5, 32, False),
     (70, 62, 49, 4, 32, False), (20, 87, 51, 5, 32, True), (3, 60, 89, 5, 64, False), (34, 85, 96, 6, 64, True),
     (70, 83, 95, 6, 32, False), (5, 49, 128, 4, 32, True), (3, 60, 130, 3, 64, False)])
 def test_equals_one_step_per_pass(gpu, sites, nx, ny, nz, precision, pool):
