@@ -876,7 +876,7 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
         if (flat || casim::resident_ok(d, d->box ? M : k_steps)) {
             for (int32_t left = k_steps; left > 0;) {
                 // with a box, a launch covers the steps between two of its own
-                const int32_t kc = d->box ? M : std::min(left, (int32_t)2048);
+                const int32_t kc = d->box ? M : std::min(left, (int32_t)(flat ? 2048 : casim::resident_most(d)));
                 left -= kc;
                 flat ? casim::site2d_steps(d, dt, kc) : casim::resident_steps(d, dt, kc);
                 if (d->box) {  // box step on the accumulated effluxes, then the rim

@@ -153,10 +153,12 @@ void sweep2_launch_f32_2d(CasimDyad *d, double dt);
 
 namespace casim {
 // Steps with the state on the chip (resident.hip).  resident_ok: the handle's
-// configuration has them (makes the plan at the first call); resident_steps: k
-// steps in one launch on the handle's stream, the buffers flipped once;
-// resident_check: throws when a launch gave up waiting.
+// configuration has them (makes the plan at the first call); resident_most: the
+// steps that one launch takes at most; resident_steps: k steps in one launch on
+// the handle's stream, the buffers flipped once; resident_check: throws when a
+// launch gave up waiting.
 bool resident_ok(CasimDyad *d, int k_steps);
+int resident_most(const CasimDyad *d);
 void resident_steps(CasimDyad *d, double dt, int k);
 void resident_check(const CasimDyad *d);
 void resident_free(CasimDyad *d);

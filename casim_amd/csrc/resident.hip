@@ -994,6 +994,15 @@ bool resident_ok(CasimDyad *d, int K) {
     return pays();
 }
 
+// Steps of one launch: at most 2048, and about half a second on the chip, far
+// below the limit of a wait, since a slab whose partners found every CU taken
+// by another handle's launch waits until that one ends.
+int resident_most(const CasimDyad *d) {
+    const Resident &r = *d->res;
+    const double rounds = (d->P.S + r.a.groups - 1) / r.a.groups;
+    return (int)std::min(2048.0, std::max(16.0, 5e5 / (rounds * (r.f->us0 + r.f->us1 * r.f->PL))));
+}
+
 void resident_steps(CasimDyad *d, double dt, int k) {
     ResArgs a = d->res->a;
     const Channels &c = d->Ch;
