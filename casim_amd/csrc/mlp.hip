@@ -426,7 +426,7 @@ __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float
 // the batch as k (frag_at's order: a wave's 32 x 16 results are one block of
 // 1 KiB), and dZ in FP32, rows first, for the bias gradients.
 // k_train_weights: a 64 x 64 tile of a layer's dW = X^T dZ, or the column sums
-// of dZ for 256 biases, and Adam on what it formed: weights, moments, the BF16
+// of dZ for 64 biases, and Adam on what it formed: weights, moments, the BF16
 // copy and its transposed copy for the next forward pass.
 //
 // Per element the operations and their order are those of k_gather, k_gemm,
@@ -477,11 +477,12 @@ __device__ __forceinline__ uint64_t pack4(const uint16_t (&h)[4]) {
 
 // Latency-bound: 32 workgroups per member at 1024 rows, each a chain of 2 depth
 // + 1 layers of eight MFMA pairs per wave between barriers, weights fetched a
-// layer ahead.  Five members, 1024 rows, width 256, depth 4: 34 us; 49 with the
+// layer ahead.  Five members, 1024 rows, width 256, depth 4: 32 us; 49 with the
 // weights in plain rows.
 __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t H[2][IMR][IMAXW + IPADK];
     __shared__ int src[IMR];
+    __shared__ float ty[IMR];
     const int unit = chiplet_unit(a.tiles * a.mg);
     if (unit < 0) return;
     const int e = unit / a.tiles, tile = unit - e * a.tiles, m0 = tile * IMR;
@@ -522,7 +523,10 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
     bf16x8_t bw[IMAXW / 32], bn[IMAXW / 32];
     float bias, bias_n = 0.f;
     forward_w(0, bw, bias);
-    if (t < IMR) src[t] = m0 + t < a.B ? a.perm[(size_t)e * a.rows + m0 + t] : -1;
+    if (t < IMR) {
+        const int r = src[t] = m0 + t < a.B ? a.perm[(size_t)e * a.rows + m0 + t] : -1;
+        ty[t] = r >= 0 ? a.Y[r] : 0.f;
+    }
     __syncthreads();
     const int kp0 = a.kp[0];
     for (int i = t; i < IMR * kp0; i += 64 * IWAVES) {
@@ -582,7 +586,7 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
             for (int r = 0; r < 4; ++r) {
                 const int row = i * 16 + rq + r;
                 const bool on = m0 + row < a.B;
-                const float er = on ? target_error(acc[i][r] + bias, a.Y[src[row]], a.ym, a.yis) : 0.f;
+                const float er = on ? target_error(acc[i][r] + bias, ty[row], a.ym, a.yis) : 0.f;
                 const float d = on ? 2.f * er / (float)a.B : 0.f;
                 if ((l & 15) == 0) DZ[(size_t)row * a.zcols + a.zcol[last]] = d;
                 h[r] = f2bf(d);
@@ -627,12 +631,14 @@ __global__ __launch_bounds__(64 * IWAVES) void k_train_rows(const TrainArgs a) {
     }
 }
 
-// Latency-bound as well (the same shape: 31 us, 41 with X and dZ in rows of the
-// batch, of which a load takes 16 half lines): a wave holds a 32 x 32 quarter of its tile and walks
+// Latency-bound as well: a wave holds a 32 x 32 quarter of its tile and walks
 // the batch in blocks of 32, TKU blocks' operands in flight; a column sum is a
-// chain of B dependent additions per lane with as many rows in flight.
-constexpr int TKU = 4, TSR = 32;
-static_assert(IMR == 32 && IMR % TSR == 0, "a row tile is one block of a weight gradient's k");
+// chain of B dependent additions, so a workgroup takes 64 columns and keeps the
+// next TSR rows on their way.  The same shape: 20 us; 33 with a lane fetching
+// its own column, 41 with X and dZ in rows of the batch besides, of which a load
+// takes 16 half lines.
+constexpr int TKU = 4, TSR = 128;
+static_assert(IMR == 32 && TSR / 4 == IMR, "a row tile is one block of a weight gradient's k and one wave's rows of a column sum");
 __global__ __launch_bounds__(256) void k_train_weights(const TrainArgs a) {
     const int ue = a.nsum + a.tile0[a.nl], unit = chiplet_unit(ue * a.mg);
     if (unit < 0) return;
@@ -642,22 +648,27 @@ __global__ __launch_bounds__(256) void k_train_weights(const TrainArgs a) {
     float *const p = a.p[e], *const am = a.am[e], *const av = a.av[e];
     uint16_t *const wt = a.wt[e];
     if (ub < a.nsum) {
-        const int col = ub * 256 + t;
-        if (col >= a.zcols) return;
-        const float *x = a.DZ + (size_t)e * a.tiles * IMR * a.zcols + col;
-        float s = 0.f, cur[TSR], nxt[TSR];
+        // 64 columns: the four waves bring in TSR rows at a time, the first adds them
+        __shared__ float rows[2][TSR][64];
+        const int col = ub * 64 + l, nr = a.tiles * IMR;  // rows past the batch hold zeros
+        const float *x = a.DZ + (size_t)e * nr * a.zcols + min(col, a.zcols - 1);
+        float s = 0.f, v[TSR / 4];
+        auto load = [&](int r0) {
+            const int r = r0 + w * (TSR / 4);
 #pragma unroll
-        for (int q = 0; q < TSR; ++q) cur[q] = x[(size_t)q * a.zcols];
-        const int nr = a.tiles * IMR;  // rows past the batch hold zeros
-        for (int r0 = 0; r0 < nr; r0 += TSR) {
-            const int r1 = r0 + TSR < nr ? r0 + TSR : r0;
+            for (int q = 0; q < TSR / 4; ++q) v[q] = r < nr ? x[(size_t)(r + q) * a.zcols] : 0.f;
+        };
+        load(0);
+        for (int r0 = 0, b = 0; r0 < nr; r0 += TSR, b ^= 1) {
 #pragma unroll
-            for (int q = 0; q < TSR; ++q) nxt[q] = x[(size_t)(r1 + q) * a.zcols];
-#pragma unroll
-            for (int q = 0; q < TSR; ++q) s += cur[q];
-#pragma unroll
-            for (int q = 0; q < TSR; ++q) cur[q] = nxt[q];
+            for (int q = 0; q < TSR / 4; ++q) rows[b][w * (TSR / 4) + q][l] = v[q];
+            __syncthreads();
+            load(r0 + TSR);
+            if (w == 0)
+#pragma unroll 16
+                for (int q = 0; q < TSR; ++q) s += rows[b][q][l];
         }
+        if (w != 0 || col >= a.zcols) return;
         int L = 0;
         while (L + 1 < a.nl && col >= a.zcol[L + 1]) ++L;
         const int q = a.boff[L] + (col - a.zcol[L]);
@@ -1067,7 +1078,7 @@ void CasimMLP::train_group(int e0, int mg, int epochs, int B, float lr, uint64_t
     }
     a.nl = depth + 1;
     a.mg = mg;
-    a.nsum = (a.zcols + 255) / 256;
+    a.nsum = (a.zcols + 63) / 64;
     a.n_in = n_in;
     a.B = B;
     a.tiles = (B + IMR - 1) / IMR;
