@@ -1509,7 +1509,12 @@ int casim_mlp_predict(CasimMLP *m, const float *x, int64_t rows, float *mean, fl
     return guard([&] {
         REQUIRE(m && x && rows >= 1, CASIM_E_INVALID, "bad arguments");
         m->use();
-        const int chunk = (int)std::min<int64_t>(rows, PREDICT_ROWS), E = m->members;
+        const int E = m->members;
+        // halved where a row is wide, so that a slot stays within 32 MiB of pinned
+        // memory (from about 500 features on; 256 rows at the least)
+        int most = PREDICT_ROWS;
+        while (most > 256 && (int64_t)most * ((int64_t)m->n_in + E + 2) > (8 << 20)) most /= 2;
+        const int chunk = (int)std::min<int64_t>(rows, most);
         const bool fused = m->fused_ok();
         if (!fused) m->reserve(chunk);
         m->predict_reserve(chunk);
