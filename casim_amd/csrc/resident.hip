@@ -921,7 +921,35 @@ struct Resident {
     ResArgs a{};
     double *kin = nullptr;
     size_t lds = 0;
+    bool ready = false;
 };
+
+// What the kernel keeps between launches, made before the first of them: a call
+// that stays with the sweeps allocates nothing.
+static void resident_buffers(CasimDyad *d, Resident &res) {
+    const bool flat = res.f->flat;
+    ResArgs &a = res.a;
+    const size_t flags = (size_t)a.units * 32 * sizeof(unsigned);
+    HIPCK(hipMalloc(&a.mflag, flags));
+    HIPCK(hipMalloc(&a.eflag, flags));
+    HIPCK(hipMalloc(&a.ticket, sizeof(*a.ticket)));
+    HIPCK(hipMalloc(&a.edge, (size_t)a.units * RES_PAR * 2 * (flat ? 4 : 3) * res.f->PS * d->tsize));
+    HIPCK(hipMalloc(&a.mouth, (size_t)a.groups * RES_PAR * RES_CH * sizeof(double)));
+    HIPCK(hipHostMalloc((void **)&a.err, sizeof(int), hipHostMallocMapped));
+    *a.err = 0;
+    std::vector<double> kin((size_t)MAXT * (NPAR + 1));
+    for (int t = 0; t < MAXT; ++t) {
+        for (int q = 0; q < NPAR; ++q) kin[t * (NPAR + 1) + q] = d->Ch.par[t * NPAR + q];
+        kin[t * (NPAR + 1) + NPAR] = d->Ch.g[t * MAXI];
+    }
+    HIPCK(hipMalloc(&res.kin, sizeof(double) * kin.size()));
+    HIPCK(hipMemcpyAsync(res.kin, kin.data(), sizeof(double) * kin.size(), hipMemcpyHostToDevice, d->stream));
+    HIPCK(hipStreamSynchronize(d->stream));  // kin is a local
+    HIPCK(hipMemsetAsync(a.mflag, 0, flags, d->stream));
+    HIPCK(hipMemsetAsync(a.eflag, 0, flags, d->stream));
+    HIPCK(hipMemsetAsync(a.ticket, 0, sizeof(*a.ticket), d->stream));
+    res.ready = true;
+}
 
 // The call pays for the load and the write-out of the state once, K steps share
 // it.  Both sides in us per call, measured over 1 to 4096 sites and 1 to 100
@@ -941,7 +969,19 @@ bool resident_ok(CasimDyad *d, int K) {
     if (!d->chan_small || (d->Q.on && d->Q.cyto) || d->steps_per_pass < 2 || !d->use_sweep || d->M >= RES_CH) return false;
     if (flat ? layout_id(p) != 2 || !box_links(d, nullptr) : d->box || layout_id(p) != 1 || p.nz < 2 || p.ny > RES_CH)
         return false;
-    if (d->res_tried) return d->res != nullptr && pays();
+    // a failed allocation leaves no plan behind, and the next call makes it anew
+    auto buffers = [&] {
+        if (d->res->ready) return true;
+        try {
+            resident_buffers(d, *d->res);
+        } catch (...) {
+            resident_free(d);
+            d->res_tried = false;
+            throw;
+        }
+        return true;
+    };
+    if (d->res_tried) return d->res != nullptr && pays() && buffers();
     d->res_tried = true;
     const int N = p.nx - 2, P = p.ny * p.nz;
     auto lds_of = [&](const Form &f) { return f.lds + (flat ? 0 : (size_t)(f.PL | 1) * 2 * p.ny * d->tsize); };
@@ -972,26 +1012,7 @@ bool resident_ok(CasimDyad *d, int K) {
     a.groups = std::min(p.S, RES_CUS / bg);
     a.units = a.groups * bg;
     a.nw = ((flat ? 2 * P + 36 : P) + 63) / 64;
-    const size_t flags = (size_t)a.units * 32 * sizeof(unsigned);
-    HIPCK(hipMalloc(&a.mflag, flags));
-    HIPCK(hipMalloc(&a.eflag, flags));
-    HIPCK(hipMalloc(&a.ticket, sizeof(*a.ticket)));
-    HIPCK(hipMalloc(&a.edge, (size_t)a.units * RES_PAR * 2 * (flat ? 4 : 3) * best->PS * d->tsize));
-    HIPCK(hipMalloc(&a.mouth, (size_t)a.groups * RES_PAR * RES_CH * sizeof(double)));
-    HIPCK(hipHostMalloc((void **)&a.err, sizeof(int), hipHostMallocMapped));
-    *a.err = 0;
-    std::vector<double> kin((size_t)MAXT * (NPAR + 1));
-    for (int t = 0; t < MAXT; ++t) {
-        for (int q = 0; q < NPAR; ++q) kin[t * (NPAR + 1) + q] = d->Ch.par[t * NPAR + q];
-        kin[t * (NPAR + 1) + NPAR] = d->Ch.g[t * MAXI];
-    }
-    HIPCK(hipMalloc(&res->kin, sizeof(double) * kin.size()));
-    HIPCK(hipMemcpyAsync(res->kin, kin.data(), sizeof(double) * kin.size(), hipMemcpyHostToDevice, d->stream));
-    HIPCK(hipStreamSynchronize(d->stream));  // kin is a local
-    HIPCK(hipMemsetAsync(a.mflag, 0, flags, d->stream));
-    HIPCK(hipMemsetAsync(a.eflag, 0, flags, d->stream));
-    HIPCK(hipMemsetAsync(a.ticket, 0, sizeof(*a.ticket), d->stream));
-    return pays();
+    return pays() && buffers();
 }
 
 // Steps of one launch: at most 2048, and about half a second on the chip, far
@@ -1024,7 +1045,7 @@ void resident_steps(CasimDyad *d, double dt, int k) {
 }
 
 void resident_check(const CasimDyad *d) {
-    if (d->res && *(volatile int *)d->res->a.err)
+    if (d->res && d->res->ready && *(volatile int *)d->res->a.err)
         throw Err(CASIM_E_DEVICE, "a step kernel gave up waiting for a workgroup of its site; the state is invalid");
 }
 

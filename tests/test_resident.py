@@ -87,6 +87,17 @@ def test_equals_one_step_per_pass(gpu, sites, nx, ny, nz, precision, pool):
     same(state(a, sp, pool), state(b, sp, pool))
 
 
+# a call too short to pay takes the sweeps and keeps nothing; longer and short
+# ones after it, in either order
+def test_short_calls_before_and_between_long_ones(gpu):
+    sp = spec(600, 52, 50, 5, abi.CASIM_FP64)
+    a, b = start(sp, False, 2), start(sp, False, 1)
+    for k in (2, 2, 60, 2, 60):
+        a.Step(1e-5, k)
+        b.Step(1e-5, k)
+    same(state(a, sp, False), state(b, sp, False))
+
+
 def test_two_handles_step_beside_each_other(gpu):
     """Launches of two handles share the chip: more workgroups than fit."""
     sp = spec(60, 81, 81, 5, abi.CASIM_FP64)
