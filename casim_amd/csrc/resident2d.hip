@@ -633,11 +633,16 @@ void site2d_plan(CasimDyad *d) {
         HIPCK(hipMalloc(&dst, sizeof(src[0]) * src.size()));
         HIPCK(hipMemcpyAsync(dst, src.data(), sizeof(src[0]) * src.size(), hipMemcpyHostToDevice, d->stream));
     };
-    up(r->kin, kin);
-    up(r->cb, cb);
-    up(r->ctot, ct);
-    up(r->ci, ci);
-    HIPCK(hipStreamSynchronize(d->stream));  // the sources are locals
+    try {
+        up(r->kin, kin);
+        up(r->cb, cb);
+        up(r->ctot, ct);
+        up(r->ci, ci);
+        HIPCK(hipStreamSynchronize(d->stream));  // the sources are locals
+    } catch (...) {  // no plan without its tables: the next call makes it anew
+        site2d_free(d);
+        throw;
+    }
 }
 
 }  // namespace
