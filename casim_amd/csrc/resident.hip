@@ -647,7 +647,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
         auto lane_states = [&](const uint32_t(&S6)[6]) {
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
-                if (64 * c >= n) break;
+                if (c && 64 * c >= n) break;  // the first chunk holds the stream, also of a site without channels
                 uint32_t o[6];
                 const uint32_t *J = r.jump + (size_t)(lane + 64 * c) * 18;
                 mrg::matvec(J, S6, o, mrg::C1, mrg::M1);
@@ -695,7 +695,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
             if (pos == n) {
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    if (64 * c >= n) break;
+                    if (c && 64 * c >= n) break;
                     jump53(S.jn, L6[c]);
                 }
             } else {

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(NT) void k_site2d(const T *__restrict__ gin, T *__r
         auto lane_states = [&](const uint32_t(&S6)[6]) {
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
-                if (64 * c >= n) break;
+                if (c && 64 * c >= n) break;  // the first chunk holds the stream, also of a site without channels
                 uint32_t o[6];
                 const uint32_t *J = a.jump + (size_t)(lane + 64 * c) * 18;
                 mrg::matvec(J, S6, o, mrg::C1, mrg::M1);
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(NT) void k_site2d(const T *__restrict__ gin, T *__r
             if (pos == n) {
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    if (64 * c >= n) break;
+                    if (c && 64 * c >= n) break;
                     jump53(S.jn, L6[c]);
                 }
             } else {
