@@ -813,10 +813,10 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
         for (int k = 0; k < r.K; ++k) {
             bool gated = false;
             bool out = k + 1 == r.K || r.G == 1;  // the neighbours' edge planes of the next step are out
-            auto look = [&] {
+            auto look = [&] {  // every lane stores: a branch on the lane here would make the loop's control flow per lane
                 if (!out && flags_out(ewatch, E + k + 1)) {
                     out = true;
-                    if (lane == 0) *(volatile unsigned *)&S.ready = E + k + 1;
+                    *(volatile unsigned *)&S.ready = E + k + 1;
                 }
             };
 #pragma unroll 1
