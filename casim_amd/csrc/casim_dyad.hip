@@ -148,12 +148,7 @@ void CasimDyad::sync() {
 }
 
 double *CasimDyad::pinned() {
-    if (!pin) {
-        HIPCK(hipHostMalloc((void **)&pin, sizeof(double) * PIN, hipHostMallocDefault));
-        HIPCK(hipEventCreateWithFlags(&pin_busy, hipEventDisableTiming));
-    } else {
-        HIPCK(hipEventSynchronize(pin_busy));
-    }
+    if (!pin) HIPCK(hipHostMalloc((void **)&pin, sizeof(double) * PIN, hipHostMallocDefault));
     return pin;
 }
 
@@ -571,7 +566,6 @@ int casim_dyad_destroy(CasimDyad *d) {
     casim::resident_free(d);
     casim::site2d_free(d);
     if (d->pin) (void)hipHostFree(d->pin);
-    if (d->pin_busy) (void)hipEventDestroy(d->pin_busy);
     void *ptrs[] = {d->g[0], d->g[1], d->f[0], d->f[1], d->d_off, d->d_node, d->d_type, d->d_perm, d->d_snode,
                     d->d_sperm, d->d_state, d->d_chans, d->d_rng, d->d_rng0, d->d_jump, d->d_mouths, d->d_sJ,
                     d->d_snap, d->d_pg, d->d_pjv, d->d_totals, d->d_rim_ions, d->d_eff, d->d_stats, d->Ch.trace};
@@ -659,14 +653,14 @@ int casim_dyad_update(CasimDyad *d, const double *rim_ions, const double *rim_bo
         const bool rim = !pool_rim && !box_rim, chan = !d->Q.on && d->M;
         const size_t ni = (size_t)P.ni * P.S, nb = (size_t)P.nb * P.S, nj = ni * d->M;
         const bool staged = rim && chan && ni + nb + nj <= CasimDyad::PIN;
+        std::unique_lock<std::mutex> lock(d->pin_mutex, std::defer_lock);
         if (staged) {
-            std::lock_guard<std::mutex> lock(d->pin_mutex);
+            lock.lock();  // until the copy is done
             double *h = d->pinned();
             std::memcpy(h, rim_ions, sizeof(double) * ni);
             if (nb) std::memcpy(h + ni, rim_bound, sizeof(double) * nb);
             std::memcpy(h + ni + nb, jsr, sizeof(double) * nj);
             HIPCK(hipMemcpyAsync(d->d_rim_ions, h, sizeof(double) * (ni + nb + nj), hipMemcpyHostToDevice, d->stream));
-            HIPCK(hipEventRecord(d->pin_busy, d->stream));
         } else {
             if (rim) {
                 HIPCK(hipMemcpyAsync(d->d_rim_ions, rim_ions, sizeof(double) * ni, hipMemcpyHostToDevice, d->stream));
@@ -683,8 +677,7 @@ int casim_dyad_update(CasimDyad *d, const double *rim_ions, const double *rim_bo
         d->launch_efflux();
         d->launch_channels(CH_SNAPSHOT | CH_CURRENTS | CH_ACCUMULATE | CH_POOL_UPDATE, 0.0);
         d->clear_graphs();
-        // the caller's arrays are free: copied to the pinned buffer, or by now to the device
-        if (!staged) HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         d->have_update = true;
     });
 }
@@ -849,7 +842,8 @@ int casim_dyad_run_rd(CasimDyad *d, double dt, int32_t site) {
         REQUIRE(d->have_update, CASIM_E_STATE, "run_rd before the first update");
         REQUIRE(!d->box, CASIM_E_STATE, "with a cytosol box, advance with casim_dyad_step");
         d->use();
-        d->launch_step(dt);  // what reads the state waits for the stream
+        d->launch_step(dt);
+        d->sync();
     });
 }
 
@@ -860,6 +854,7 @@ int casim_dyad_run_mc(CasimDyad *d, double dt, int32_t site) {
         REQUIRE(d->have_update, CASIM_E_STATE, "run_mc before the first update");
         d->use();
         d->launch_channels(CH_GATE_STORED, dt);
+        d->sync();
     });
 }
 

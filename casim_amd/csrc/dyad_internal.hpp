@@ -100,10 +100,9 @@ struct CasimDyad {
     casim::Site2D *s2d = nullptr;
     // Pinned buffer for small transfers (the update's inputs, site values): a
     // copy from or to pageable memory is staged by the runtime, which waits for
-    // it.  pinned(): the buffer, free for use, with pin_mutex held.
+    // it.  pinned(): the buffer; a call holds pin_mutex until its copy is done.
     static constexpr size_t PIN = (size_t)1 << 17;  // doubles
     double *pin = nullptr;
-    hipEvent_t pin_busy = nullptr;
     std::mutex pin_mutex;
     double *pinned();
     // the sites and stream the pair and channel launchers work on (all sites
