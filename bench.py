@@ -1,8 +1,9 @@
 """Batched dyad reaction-diffusion benchmark (one GPU).
 
-A "step" advances every site of the batch by one dt: channel kernel (mouth
-snapshot, RyR currents, stochastic gating) + the fused state sweep, replayed
-from a captured HIP graph.  Inputs are resident in HBM before timing starts.
+A "step" advances every site of the batch by one dt: mouth snapshot, RyR
+currents, stochastic gating and the state update, by whatever casim_dyad_step
+takes for calls of --chunk steps (the path is reported).  Inputs are resident in
+HBM before timing starts.
 
 Workload: 4096 independent release sites, 81 x 81 x 5 nodes each (320 x 320 x
 16 nm at h = 4 nm), free Ca2+ + ATP-like + calmodulin-like mobile buffers +
@@ -55,7 +56,7 @@ def run_gpu_leg(workloads, DyadHIP, precision, n_sites, steps, warmup, chunk, re
     log("tuning:", {k: tuned[k] for k in ("planes", "threads", "sweep_ms")})
     chunk = min(chunk, steps)
     rem = steps % chunk
-    # warmup also captures the graphs used in the timed region
+    # warmup also captures the graphs, or makes the buffers, of the timed region
     done = 0
     while done < max(warmup, 1):
         dev.Step(dt, chunk)
@@ -66,6 +67,7 @@ def run_gpu_leg(workloads, DyadHIP, precision, n_sites, steps, warmup, chunk, re
     t0 = time.perf_counter()
     for _ in range(steps // chunk):
         dev.Step(dt, chunk)
+    path = dev.StepPath()
     if rem:
         dev.Step(dt, rem)
     dev.Synchronize()
@@ -87,7 +89,7 @@ def run_gpu_leg(workloads, DyadHIP, precision, n_sites, steps, warmup, chunk, re
         "dyad_ms_per_s": n_sites * steps * dt / t,
         "bytes_per_site_step": bps,
         "sweep_kernel_ms": ms_sweep / steps, "channel_kernel_ms": ms_chan / steps,
-        "steps_per_launch": per_pass, "sweep_launch_ms": ms_sweep / launches,
+        "step_path": path, "steps_per_launch": per_pass, "sweep_launch_ms": ms_sweep / launches,
         # one read and one write of the state per launch, whatever the steps it advances
         "sweep_gbs": n_sites * bps / (ms_sweep / launches * 1e-3) / 1e9,
         "finite": ok, "open_fraction": open_frac,
@@ -256,6 +258,45 @@ def coupled_leg(workloads, DyadHIP, n_sites, steps, warmup, chunk=100, tuning=No
     return res
 
 
+def plain_leg_figures(r, abi):
+    """(roofline, sweep figures, path, whole-step GB/s) of a plain leg, by what
+    its calls ran."""
+    on_chip = r["step_path"] == abi.CASIM_STEP_SLABS
+    # sweep kernels: k_sweep2 (two steps per launch) or k_sweep (one).  Their
+    # algorithmic bytes per launch are one read and one write of every
+    # site's state (sites x bytes per site-step): a two-step launch moves the
+    # state once, so the steps it advances do not multiply the bytes.
+    kernel = "k_sweep2" if r["steps_per_launch"] == 2 else "k_sweep"
+    launch_bytes = r["sites"] * r["bytes_per_site_step"]
+    achieved = launch_bytes / (r["sweep_launch_ms"] * 1e-3) / 1e9
+    traffic = traffic_from_profiles(kernel)
+    sweep = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
+             "kernel": kernel, "steps_per_launch": r["steps_per_launch"],
+             "launch_ms": r["sweep_launch_ms"], "algorithmic_bytes_per_launch": launch_bytes,
+             # what HBM actually moves per launch (traffic / launch time), next to the copy rate
+             "physical_gbs": None if traffic is None else traffic / (r["sweep_launch_ms"] * 1e-3) / 1e9,
+             "copy_gbs": COPY_GBS,
+             # per-step algorithmic rate: the bytes a one-step-per-pass sweep would move
+             # for the same steps, over the same time (not bounded by the HBM peak)
+             "effective_gbs": r["steps_per_launch"] * achieved}
+    if not on_chip:
+        # one-step-per-pass bytes of a whole step (channels + sweep) over its time
+        whole = launch_bytes / (r["ms_per_step"] * 1e-3) / 1e9
+        path = "two steps per state pass" if r["steps_per_launch"] == 2 else "one step per pass"
+        return sweep, sweep, path, whole
+    # k_resident, the state in registers over a call's steps: bound by FP64 issue,
+    # LDS and the barriers of a step, so priced in operations: per interior node 14
+    # for each of the three diffusing fields and 9 for each bound field (the third
+    # on the two z-faces only).  No step moves the state, so there is no rate of it.
+    nx, ny, nz = (int(v) for v in r["grid"].split("x"))
+    flops = (nx - 2) * (ny - 2) * (nz * (3 * 14 + 2 * 9) + 2 * 9)
+    tflops = r["sites"] * flops / (r["ms_per_step"] * 1e-3) / 1e12
+    return ({"bound": "fp64", "achieved": tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+             "frac": tflops / FP64_PEAK_TFLOPS, "kernel": "k_resident", "flops_per_site_step": flops},
+            sweep, "state on the chip", None)
+
+
 def traffic_from_profiles(kernel):
     """HBM bytes per sweep-kernel launch from the committed rocprofv3 --pmc
     summary (FETCH_SIZE + WRITE_SIZE, KiB, scaled by the copy-kernel factor)."""
@@ -275,7 +316,7 @@ def main():
     ap.add_argument("--steps", type=int, default=400)
     ap.add_argument("--warmup", type=int, default=100)
     ap.add_argument("--sites", type=int, default=4096)
-    ap.add_argument("--chunk", type=int, default=100, help="steps per captured HIP graph")
+    ap.add_argument("--chunk", type=int, default=100, help="steps per call")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-fp32", action="store_true")
     ap.add_argument("--retune", action="store_true", help="ignore the tuning cache")
@@ -330,33 +371,7 @@ def main():
         log("cpu baseline")
         cpu = cpu_baseline(workloads)
         log("cpu:", json.dumps(cpu))
-    # dominant kernel: k_resident, the state in registers over a call's steps;
-    # bound by FP64 issue and the barriers of a step, so priced in operations:
-    # per interior node 14 for each of the three diffusing fields and 9 for each
-    # bound field (the third on the two z-faces only).  With one step per pass
-    # the sweep takes its place.
-    resident = a.steps_per_pass == 2
-    nx, ny, nz = (int(v) for v in r64["grid"].split("x"))
-    flops = (nx - 2) * (ny - 2) * (nz * (3 * 14 + 2 * 9) + 2 * 9)
-    tflops = a.sites * flops / (r64["ms_per_step"] * 1e-3) / 1e12
-    # sweep kernels: k_sweep2 (two steps per launch) or k_sweep (one).  Their
-    # algorithmic bytes per launch are one read and one write of every
-    # site's state (sites x bytes per site-step): a two-step launch moves the
-    # state once, so the steps it advances do not multiply the bytes.
-    kernel = "k_sweep2" if r64["steps_per_launch"] == 2 else "k_sweep"
-    launch_bytes = a.sites * r64["bytes_per_site_step"]
-    achieved = launch_bytes / (r64["sweep_launch_ms"] * 1e-3) / 1e9
-    traffic = traffic_from_profiles(kernel)
-    sweep = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-             "kernel": kernel, "steps_per_launch": r64["steps_per_launch"],
-             "launch_ms": r64["sweep_launch_ms"], "algorithmic_bytes_per_launch": launch_bytes,
-             # what HBM actually moves per launch (traffic / launch time), next to the copy rate
-             "physical_gbs": None if traffic is None else traffic / (r64["sweep_launch_ms"] * 1e-3) / 1e9,
-             "copy_gbs": COPY_GBS,
-             # per-step algorithmic rate: the bytes a one-step-per-pass sweep would move
-             # for the same steps, over the same time (not bounded by the HBM peak)
-             "effective_gbs": r64["steps_per_launch"] * achieved}
+    roofline, sweep, path, effective = plain_leg_figures(r64, abi)
     out = {
         "metric": METRIC,
         "value": r64["dyad_ms_per_s"],
@@ -371,16 +386,12 @@ def main():
         "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": r64["workload"], "sites": a.sites, "grid": r64["grid"], "dt_ns": 10,
-                   "path": "plain batched RD, calls of %d steps%s" % (
-                       min(a.chunk, a.steps), ", state on the chip" if resident else ", one step per pass"),
+                   "path": "plain batched RD, calls of %d steps, %s" % (min(a.chunk, a.steps), path),
                    "tuning": r64["tuning"]},
-        "roofline": {"bound": "fp64", "achieved": tflops, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": tflops / FP64_PEAK_TFLOPS, "kernel": "k_resident",
-                     "flops_per_site_step": flops} if resident else sweep,
+        "roofline": roofline,
         "sweep": sweep,
         "cpu_baseline": cpu,
-        # one-step-per-pass bytes of a whole step (channels + sweep) over its time
-        "effective_gbs_whole_step": a.sites * r64["bytes_per_site_step"] / (r64["ms_per_step"] * 1e-3) / 1e9,
+        "effective_gbs_whole_step": effective,
         "fp32": None if r32 is None else {
             "value": r32["dyad_ms_per_s"], "ms_per_step": r32["ms_per_step"], "sweep_gbs": r32["sweep_gbs"],
             "sweep_kernel_ms": r32["sweep_kernel_ms"]},

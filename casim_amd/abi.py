@@ -16,6 +16,7 @@ CASIM_MODEL_TWO_STATE_MWC = 2
 CASIM_MODEL_TWO_STATE_AHTG = 3
 CASIM_MAX_MODEL_PARAMS = 16
 CASIM_E_INVALID, CASIM_E_DEVICE, CASIM_E_STATE, CASIM_E_RANGE = -1, -2, -3, -4
+CASIM_STEP_PASSES, CASIM_STEP_SLABS, CASIM_STEP_SITE = 1, 2, 3
 CASIM_FP64 = 0
 CASIM_FP32 = 1
 
@@ -107,6 +108,7 @@ def _declare(lib):
         "casim_dyad_run_rd": (C.c_int, [P, C.c_double, C.c_int32]),
         "casim_dyad_run_mc": (C.c_int, [P, C.c_double, C.c_int32]),
         "casim_dyad_step": (C.c_int, [P, C.c_double, C.c_int32]),
+        "casim_dyad_step_path": (C.c_int32, [P, _ip]),
         "casim_dyad_step_profiled": (C.c_int, [P, C.c_double, C.c_int32, _dp]),
         "casim_dyad_synchronize": (C.c_int, [P]),
         "casim_dyad_get_effluxes": (C.c_int, [P, _dp]),

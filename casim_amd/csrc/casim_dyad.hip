@@ -868,11 +868,14 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
                 "with a cytosol box, k_steps must be a multiple of its substeps");
         d->use();
         const bool flat = casim::site2d_ok(d);
+        d->step_launch = 0;
         if (flat || casim::resident_ok(d, d->box ? M : k_steps)) {
+            d->step_path = flat ? CASIM_STEP_SITE : CASIM_STEP_SLABS;
             for (int32_t left = k_steps; left > 0;) {
                 // with a box, a launch covers the steps between two of its own
                 const int32_t kc = d->box ? M : std::min(left, (int32_t)(flat ? 2048 : casim::resident_most(d)));
                 left -= kc;
+                d->step_launch = std::max(d->step_launch, (int)kc);
                 flat ? casim::site2d_steps(d, dt, kc) : casim::resident_steps(d, dt, kc);
                 if (d->box) {  // box step on the accumulated effluxes, then the rim
                     casim::box_step(d, M * dt);
@@ -885,6 +888,7 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
             }
             return;
         }
+        d->step_path = CASIM_STEP_PASSES;
         // One captured graph covers at most 2048 steps, a whole number of
         // box steps: a longer call replays several graphs, which gives the
         // results of one (each graph ends with the update that the next
@@ -894,6 +898,7 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
         for (int32_t left = k_steps; left > 0;) {
             const int32_t kc = std::min(left, (int32_t)cap);
             left -= kc;
+            d->step_launch = std::max(d->step_launch, (int)kc);
             const int cur0 = d->cur, bcur0 = casim::box_cur(d);
             auto key = std::make_tuple((int)kc, dt, cur0 | bcur0 << 1);
             auto it = d->graphs.find(key);
@@ -1007,6 +1012,11 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
             casim::box_set_cur(d, bcur0 ^ (it->second.second >> 1));
         }
     });
+}
+
+int32_t casim_dyad_step_path(const CasimDyad *d, int32_t *launch_steps) {
+    if (d && launch_steps) *launch_steps = d->step_launch;
+    return d ? d->step_path : -1;
 }
 
 int casim_dyad_step_profiled(CasimDyad *d, double dt, int32_t k_steps, double kernel_ms[2]) {

@@ -109,6 +109,16 @@ class DyadHIP:
     def Step(self, dt, k):
         abi.check(self.lib.casim_dyad_step(self.h, dt, k))
 
+    def StepPath(self):
+        """What the last Step ran (abi.CASIM_STEP_*)."""
+        return self.lib.casim_dyad_step_path(self.h, None)
+
+    def StepLaunch(self):
+        """Steps of the longest launch (or graph) of the last Step."""
+        n = C.c_int32(0)
+        self.lib.casim_dyad_step_path(self.h, C.byref(n))
+        return n.value
+
     def StepProfiled(self, dt, k):
         """k fused steps launched eagerly with HIP events around each kernel;
         returns (state-sweep kernel ms, channel kernel ms) summed over k."""

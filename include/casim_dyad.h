@@ -244,6 +244,16 @@ int casim_dyad_run_mc(CasimDyad *d, double dt, int32_t site);
  */
 int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps);
 
+/* What the last casim_dyad_step of the handle ran: passes over the state
+ * (k_sweep2, k_sweep or k_step, in a graph), a site's state dealt to several
+ * workgroups (k_resident), or a workgroup per 2D site (k_site2d).  0 before the
+ * first step, -1 for a null handle.  launch_steps (may be NULL) receives the
+ * steps of its longest launch (passes: of its longest graph). */
+#define CASIM_STEP_PASSES 1
+#define CASIM_STEP_SLABS 2
+#define CASIM_STEP_SITE 3
+int32_t casim_dyad_step_path(const CasimDyad *d, int32_t *launch_steps);
+
 /* The same k_steps as casim_dyad_step, launched eagerly (no graph) with a
  * HIP event pair around every kernel on the handle's stream.  kernel_ms[0]
  * receives the summed duration of the state-sweep kernels, kernel_ms[1] that
