@@ -871,13 +871,14 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
         d->step_launch = 0;
         if (flat || casim::resident_ok(d, d->box ? M : k_steps)) {
             d->step_path = flat ? CASIM_STEP_SITE : CASIM_STEP_SLABS;
+            const int32_t most = flat ? 2048 : casim::resident_most(d);
             for (int32_t left = k_steps; left > 0;) {
-                // with a box, a launch covers the steps between two of its own
-                const int32_t kc = d->box ? M : std::min(left, (int32_t)(flat ? 2048 : casim::resident_most(d)));
+                // with a box, a launch ends at the latest where the box takes a step of its own
+                const int32_t at = d->box ? (k_steps - left) % M : 0, kc = std::min(most, d->box ? M - at : left);
                 left -= kc;
                 d->step_launch = std::max(d->step_launch, (int)kc);
-                flat ? casim::site2d_steps(d, dt, kc) : casim::resident_steps(d, dt, kc);
-                if (d->box) {  // box step on the accumulated effluxes, then the rim
+                flat ? casim::site2d_steps(d, dt, kc) : casim::resident_steps(d, dt, kc, at > 0);
+                if (d->box && at + kc == M) {  // box step on the accumulated effluxes, then the rim
                     casim::box_step(d, M * dt);
                     casim::box_rim(d);
                 }

@@ -155,11 +155,12 @@ namespace casim {
 // Steps with the state on the chip (resident.hip).  resident_ok: the handle's
 // configuration has them (makes the plan at the first call); resident_most: the
 // steps that one launch takes at most; resident_steps: k steps in one launch on
-// the handle's stream, the buffers flipped once; resident_check: throws when a
+// the handle's stream, the buffers flipped once, a box's accumulated effluxes
+// taken on from the launch before with carry; resident_check: throws when a
 // launch gave up waiting.
 bool resident_ok(CasimDyad *d, int k_steps);
 int resident_most(const CasimDyad *d);
-void resident_steps(CasimDyad *d, double dt, int k);
+void resident_steps(CasimDyad *d, double dt, int k, bool carry);
 void resident_check(const CasimDyad *d);
 void resident_free(CasimDyad *d);
 // The same for 2D sites that fit one CU (resident2d.hip).

@@ -78,6 +78,7 @@ struct ResArgs {
     double exD[3];
     const double *link_fac;
     double *acc;
+    int carry;  // the accumulator holds the effluxes of earlier launches of this box step
 };
 
 // SRPool::Update and SRPool::Run (SRPool.cpp:55-89) of one site held in
@@ -234,6 +235,11 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
         const int al = FLAT && r.ne ? q - 2 * P : -1, asub = al / 12, af = al < 0 ? 0 : (al >> 2) % 3;
         const bool acc_lane = FLAT && al >= 0 && al < 36 && af < r.ne;
         const int arim = (al & 1) * P + (al >> 1 & 1 ? P - 1 : 0), ain = arim + (al >> 1 & 1 ? -1 : 1);
+        // ... of slots i: the place in its phase, the plane, the accumulator of its side
+        const int ah0 = al & 1 ? x0 + npa : x0, ah1 = al & 1 ? x1 : x0 + npa;
+        auto acc_place = [&](int i) { return i == 0 ? 0 : i == PL - 1 ? 1 : (i - 1) % PH; };
+        auto acc_plane = [&](int i) { return i < H ? ah0 + i : ah1 - PL + i; };
+        auto acc_y = [&](int s) { return r.acc + ((size_t)af * p.S + s) * r.nlink + 2 * (P - 2) + (al >> 1 & 1) * N; };
         const double exd = FLAT ? (af == 0 ? r.exD[0] : af == 1 ? r.exD[1] : r.exD[2]) : 0.0;
         const double facx = FLAT && r.ne ? r.link_fac[0] : 0.0, facy = FLAT && r.ne ? r.link_fac[2 * (P - 2)] : 0.0;
         auto flux = [&](double v, double D, double fac, double u, double ur) {  // k_box_efflux
@@ -270,10 +276,22 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                 hl[g] = act ? ld_off(gs + g * fs, (unsigned)(((lx0 - 1) * P + yq) * (int)sizeof(T))) : (T)0;
                 hr[g] = act ? ld_off(gs + g * fs, (unsigned)((lx1 * P + yq) * (int)sizeof(T))) : (T)0;
             }
-            if (FLAT && r.ne) {
+            if (FLAT && r.ne && !r.carry) {
                 for (int i = q; i < PL * 12; i += r.nw * 64) S.yacc[i] = 0.0;
                 for (int e = 0; e < 3; ++e)
                     if (q < PS) S.xacc[e * PS + q] = 0.0;
+            }
+            if (FLAT && r.carry) {  // every lane what it adds to, from where it is written out below
+                if (acc_lane) {
+                    const double *from = acc_y(s);
+#pragma unroll 1
+                    for (int i = 0; i < PL; ++i)
+                        if (acc_place(i) % 3 == asub) S.yacc[i * 12 + al % 12] = from[acc_plane(i) - 1];
+                }
+                if (inner && (z ? gi == r.G - 1 : gi == 0))
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (e < r.ne) S.xacc[e * PS + q] = r.acc[((size_t)e * p.S + s) * r.nlink + z * (P - 2) + y - 1];
             }
             __syncthreads();  // map cleared: the channel wave enters the mouths
             __syncthreads();
@@ -545,14 +563,11 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
             T *os = gout + (size_t)s * p.NS;
             T *ofs = fout + (size_t)s * 2 * p.nFP;
             if (FLAT && acc_lane) {
-                const int h0 = al & 1 ? x0 + npa : x0, h1 = al & 1 ? x1 : x0 + npa, hd = PL - (h1 - h0);
-                double *to = r.acc + ((size_t)af * p.S + s) * r.nlink + 2 * (P - 2) + (al >> 1 & 1) * N;
+                double *to = acc_y(s);
 #pragma unroll 1
-                for (int i = 0; i < PL; ++i) {
-                    const int at = i == 0 ? 0 : i == PL - 1 ? 1 : (i - 1) % PH;  // its place in its phase
-                    if (at % 3 != asub || (i >= H && i < H + hd)) continue;
-                    to[(i < H ? h0 + i : h1 - PL + i) - 1] = S.yacc[i * 12 + al % 12];
-                }
+                for (int i = 0; i < PL; ++i)
+                    if (acc_place(i) % 3 == asub && (i < H || i >= H + PL - (ah1 - ah0)))
+                        to[acc_plane(i) - 1] = S.yacc[i * 12 + al % 12];
             }
             if (FLAT && r.ne && inner && (z ? gi == r.G - 1 : gi == 0))
 #pragma unroll
@@ -1015,17 +1030,18 @@ bool resident_ok(CasimDyad *d, int K) {
     return pays() && buffers();
 }
 
-// Steps of one launch: at most 2048, and about half a second on the chip, far
-// below the limit of a wait, since a slab whose partners found every CU taken
-// by another handle's launch waits until that one ends.
+// Steps of one launch, with a cytosol box too: at most 2048, and about half a
+// second on the chip, far below the limit of a wait, since a slab whose partners
+// found every CU taken by another handle's launch waits until that one ends.
 int resident_most(const CasimDyad *d) {
     const Resident &r = *d->res;
     const double rounds = (d->P.S + r.a.groups - 1) / r.a.groups;
     return (int)std::min(2048.0, std::max(16.0, 5e5 / (rounds * (r.f->us0 + r.f->us1 * r.f->PL))));
 }
 
-void resident_steps(CasimDyad *d, double dt, int k) {
+void resident_steps(CasimDyad *d, double dt, int k, bool carry) {
     ResArgs a = d->res->a;
+    a.carry = carry;
     const Channels &c = d->Ch;
     const Pools &q = d->Q;
     a.K = k;
