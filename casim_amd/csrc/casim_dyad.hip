@@ -634,7 +634,7 @@ int casim_dyad_init_opening(CasimDyad *d, int32_t site, int32_t channel, const i
         hipLaunchKernelGGL(k_init_opening, dim3((d->P.S + 127) / 128), dim3(128), 0, d->stream, d->Ch, d->P.S, site,
                            channel, dch);
         HIPCK(hipGetLastError());
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 
@@ -815,7 +815,7 @@ int casim_dyad_attach_pools(CasimDyad *d, const CasimPoolConfig *pc) {
         d->Q = Q;
         hipLaunchKernelGGL(k_pools_reset, dim3((S + 127) / 128), dim3(128), 0, d->stream, d->Q, S, ni, d->d_jc0);
         HIPCK(hipGetLastError());
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
         d->have_update = false;
         d->clear_graphs();
     });
@@ -867,6 +867,7 @@ int casim_dyad_step(CasimDyad *d, double dt, int32_t k_steps) {
         REQUIRE(!d->box || k_steps % M == 0, CASIM_E_INVALID,
                 "with a cytosol box, k_steps must be a multiple of its substeps");
         d->use();
+        casim::resident_check(d);
         const bool flat = casim::site2d_ok(d);
         d->step_launch = 0;
         if (flat || casim::resident_ok(d, d->box ? M : k_steps)) {
@@ -1074,7 +1075,7 @@ int casim_dyad_step_profiled(CasimDyad *d, double dt, int32_t k_steps, double ke
             if (pool_rim) d->launch_rim(d->Q.cions, d->Q.cbb);
             d->launch_efflux();
             d->launch_channels(CH_SNAPSHOT | CH_CURRENTS | CH_ACCUMULATE | CH_POOL_UPDATE, dt);
-            HIPCK(hipStreamSynchronize(d->stream));
+            d->sync();
             double ms_ch = 0, ms_st = 0;
             for (int k = 0; k < k_steps; ++k) {
                 float a = 0, b = 0;
@@ -1390,6 +1391,14 @@ int casim_dyad_set_steps_per_pass(CasimDyad *d, int32_t steps) {
 }
 
 int32_t casim_dyad_steps_per_pass(const CasimDyad *d) { return d ? (d->pair_ok() ? 2 : 1) : -1; }
+
+int casim_dyad_set_wait_limit(CasimDyad *d, double seconds) {
+    return guard([&] {
+        REQUIRE(d, CASIM_E_INVALID, "null handle");
+        REQUIRE(seconds >= 0 && seconds <= 3600, CASIM_E_INVALID, "the limit must be in 0..3600 s");
+        d->wait_limit = seconds;
+    });
+}
 
 int casim_dyad_set_split(CasimDyad *d, int32_t on) {
     return guard([&] {

@@ -673,7 +673,7 @@ int casim_dyad_get_cytosol_box(CasimDyad *d, int32_t field, double *out) {
         const size_t per = (size_t)d->P.S * d->box->a.NB;
         HIPCK(hipMemcpyAsync(out, d->box->b[d->box->cur] + field * per, sizeof(double) * per, hipMemcpyDeviceToHost,
                              d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 
@@ -687,7 +687,7 @@ int casim_dyad_set_cytosol_box(CasimDyad *d, int32_t field, const double *in) {
         for (int i = 0; i < 2; ++i)
             HIPCK(hipMemcpyAsync(d->box->b[i] + field * per, in, sizeof(double) * per, hipMemcpyHostToDevice,
                                  d->stream));
-        HIPCK(hipStreamSynchronize(d->stream));
+        d->sync();
     });
 }
 

@@ -98,6 +98,7 @@ struct CasimDyad {
     casim::Resident *res = nullptr;  // made by the first step that it can take
     bool res_tried = false;
     casim::Site2D *s2d = nullptr;
+    double wait_limit = 20.0;  // seconds that a workgroup of k_resident waits for another
     int step_path = 0, step_launch = 0;  // CASIM_STEP_* of the last casim_dyad_step, its longest launch
     // Pinned buffer for small transfers (the update's inputs, site values): a
     // copy from or to pageable memory is staged by the runtime, which waits for

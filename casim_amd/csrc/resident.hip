@@ -59,6 +59,8 @@ struct ResArgs {
     void *edge;               // T [units][RES_PAR][2][NG][PS]
     double *mouth;            // [groups][RES_PAR][RES_CH]
     int *err;                 // host-visible: set when a wait ran into its limit
+    int *stop;                // the same for later launches, which leave at once
+    long long limit;          // of a wait, in ticks of 10 ns
     // channels (see Channels; one ion)
     const int *off, *perm, *snode, *type;
     int *state;
@@ -135,15 +137,16 @@ struct ResLds {
 __device__ __forceinline__ bool flags_out(const unsigned *watch, unsigned target) {
     return !__ballot(watch && (int)(xld(watch) - target) < 0);
 }
-// Wait for them; false when the limit (20 s at 100 MHz) has passed, which only
-// a missing partner workgroup could cause.
-__device__ __forceinline__ bool wait_flags(const unsigned *watch, unsigned target) {
+// Wait for them; false when the limit has passed, which only a missing partner
+// workgroup could cause.  A limit of 0: not at all.
+__device__ __forceinline__ bool wait_flags(const unsigned *watch, unsigned target, long long limit) {
     long long t0 = 0;
     for (unsigned n = 1; !flags_out(watch, target); ++n) {
+        if (limit == 0) return false;
         if ((n & 255u) == 0) {
             const long long t = wall_clock64();
             if (!t0) t0 = t;
-            if (t - t0 > 2000000000ll) return false;
+            if (t - t0 > limit) return false;
         }
     }
     return true;
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
         S.unit = (int)(atomicAdd(r.ticket, 1ull) % (unsigned long long)r.units);
         S.base = xld(r.mflag + (size_t)S.unit * 32);
         S.ready = S.base;
-        S.abort = 0;
+        S.abort = xld(r.stop);  // the slabs of a site may stand at different steps
     }
     __syncthreads();
     const int unit = __builtin_amdgcn_readfirstlane(S.unit);
@@ -843,18 +846,19 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
                 if (j >= 1 && !gated && ok) {
                     gated = flags_out(mwatch, E + k + 1);
                     if (j >= EB) look();
-                    if (!gated && j == GL) gated = ok = wait_flags(mwatch, E + k + 1);
+                    if (!gated && j == GL) gated = ok = wait_flags(mwatch, E + k + 1, r.limit);
                     if (gated) gate(k);
                 }
                 if (j >= EB && ok) {
                     look();
                     if (!out && j == NPH - 1) {
-                        ok = wait_flags(ewatch, E + k + 1);
+                        ok = wait_flags(ewatch, E + k + 1, r.limit);
                         look();
                     }
                 }
                 if (j == NPH - 1 && !ok && lane == 0) {
                     *(volatile int *)&S.abort = 1;
+                    xst(r.stop, 1);
                     __hip_atomic_store(r.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 }
             }
@@ -939,6 +943,13 @@ struct Resident {
     bool ready = false;
 };
 
+static void clear_flags(CasimDyad *d, const ResArgs &a) {
+    const size_t flags = (size_t)a.units * 32 * sizeof(unsigned);
+    HIPCK(hipMemsetAsync(a.mflag, 0, flags, d->stream));
+    HIPCK(hipMemsetAsync(a.eflag, 0, flags, d->stream));
+    HIPCK(hipMemsetAsync(a.ticket, 0, 2 * sizeof(*a.ticket), d->stream));
+}
+
 // What the kernel keeps between launches, made before the first of them: a call
 // that stays with the sweeps allocates nothing.
 static void resident_buffers(CasimDyad *d, Resident &res) {
@@ -947,7 +958,8 @@ static void resident_buffers(CasimDyad *d, Resident &res) {
     const size_t flags = (size_t)a.units * 32 * sizeof(unsigned);
     HIPCK(hipMalloc(&a.mflag, flags));
     HIPCK(hipMalloc(&a.eflag, flags));
-    HIPCK(hipMalloc(&a.ticket, sizeof(*a.ticket)));
+    HIPCK(hipMalloc(&a.ticket, 2 * sizeof(*a.ticket)));
+    a.stop = (int *)(a.ticket + 1);
     HIPCK(hipMalloc(&a.edge, (size_t)a.units * RES_PAR * 2 * (flat ? 4 : 3) * res.f->PS * d->tsize));
     HIPCK(hipMalloc(&a.mouth, (size_t)a.groups * RES_PAR * RES_CH * sizeof(double)));
     HIPCK(hipHostMalloc((void **)&a.err, sizeof(int), hipHostMallocMapped));
@@ -960,9 +972,7 @@ static void resident_buffers(CasimDyad *d, Resident &res) {
     HIPCK(hipMalloc(&res.kin, sizeof(double) * kin.size()));
     HIPCK(hipMemcpyAsync(res.kin, kin.data(), sizeof(double) * kin.size(), hipMemcpyHostToDevice, d->stream));
     HIPCK(hipStreamSynchronize(d->stream));  // kin is a local
-    HIPCK(hipMemsetAsync(a.mflag, 0, flags, d->stream));
-    HIPCK(hipMemsetAsync(a.eflag, 0, flags, d->stream));
-    HIPCK(hipMemsetAsync(a.ticket, 0, sizeof(*a.ticket), d->stream));
+    clear_flags(d, a);
     res.ready = true;
 }
 
@@ -1042,6 +1052,7 @@ int resident_most(const CasimDyad *d) {
 void resident_steps(CasimDyad *d, double dt, int k, bool carry) {
     ResArgs a = d->res->a;
     a.carry = carry;
+    a.limit = (long long)(d->wait_limit * 1e8);
     const Channels &c = d->Ch;
     const Pools &q = d->Q;
     a.K = k;
@@ -1062,7 +1073,8 @@ void resident_steps(CasimDyad *d, double dt, int k, bool carry) {
 
 void resident_check(const CasimDyad *d) {
     if (d->res && d->res->ready && *(volatile int *)d->res->a.err)
-        throw Err(CASIM_E_DEVICE, "a step kernel gave up waiting for a workgroup of its site; the state is invalid");
+        throw Err(CASIM_E_DEVICE,
+                  "a step kernel gave up waiting for a workgroup of its site; the state is invalid (casim_dyad_reset)");
 }
 
 void resident_free(CasimDyad *d) {

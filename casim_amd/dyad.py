@@ -228,5 +228,10 @@ class DyadHIP:
         results do not depend on it."""
         abi.check(self.lib.casim_dyad_set_split(self.h, int(bool(on))))
 
+    def SetWaitLimit(self, seconds):
+        """How long a workgroup of a step with the state on the chip waits for
+        another one of its site before the launch gives up."""
+        abi.check(self.lib.casim_dyad_set_wait_limit(self.h, seconds))
+
     def stream(self):
         return self.lib.casim_dyad_stream(self.h)

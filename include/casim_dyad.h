@@ -356,6 +356,15 @@ int32_t casim_dyad_steps_per_pass(const CasimDyad *d);
  * the same bit for bit; 0 keeps one stream. */
 int casim_dyad_set_split(CasimDyad *d, int32_t on);
 
+/* Longest time, in seconds, that a workgroup of a step with the state on the
+ * chip waits for another workgroup of its site (20 by default; no counterpart in
+ * the reference).  Only something else that holds the GPU's compute units could
+ * make it wait that long; then the launch gives up, launches behind it leave at
+ * once, and every call that waits for the handle's stream, and casim_dyad_step,
+ * returns CASIM_E_DEVICE: the state is invalid.  0: no wait at all, so that
+ * nearly every such step gives up. */
+int casim_dyad_set_wait_limit(CasimDyad *d, double seconds);
+
 /*
  * 3D cytosol box around each site, coupled at the dyad's rim.  Extension:
  * the reference's coupled solver (DyadRD2DwCytosol.cu:53-59, 119-241) puts
