@@ -606,6 +606,7 @@ int casim_dyad_reset(CasimDyad *d) {
         }
         HIPCK(hipMemcpyAsync(d->d_rng, d->d_rng0, sizeof(uint32_t) * P.S * 6, hipMemcpyDeviceToDevice, d->stream));
         HIPCK(hipStreamSynchronize(d->stream));
+        casim::resident_reset(d);
         if (d->box) casim::box_reset(d);
         d->cur = 0;
         d->have_update = false;

@@ -163,6 +163,7 @@ bool resident_ok(CasimDyad *d, int k_steps);
 int resident_most(const CasimDyad *d);
 void resident_steps(CasimDyad *d, double dt, int k, bool carry);
 void resident_check(const CasimDyad *d);
+void resident_reset(CasimDyad *d);  // after such a launch, with the stream idle: ready for the next
 void resident_free(CasimDyad *d);
 // The same for 2D sites that fit one CU (resident2d.hip).
 bool site2d_ok(const CasimDyad *d);

@@ -1077,6 +1077,13 @@ void resident_check(const CasimDyad *d) {
                   "a step kernel gave up waiting for a workgroup of its site; the state is invalid (casim_dyad_reset)");
 }
 
+void resident_reset(CasimDyad *d) {
+    if (!d->res || !d->res->ready || !*(volatile int *)d->res->a.err) return;
+    clear_flags(d, d->res->a);
+    HIPCK(hipStreamSynchronize(d->stream));
+    *(volatile int *)d->res->a.err = 0;
+}
+
 void resident_free(CasimDyad *d) {
     if (!d->res) return;
     ResArgs &a = d->res->a;

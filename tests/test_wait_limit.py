@@ -8,7 +8,7 @@ import pytest
 
 from casim_amd import abi, workloads
 from casim_amd.dyad import DyadHIP
-from tests.test_resident import POOL, spec, start
+from tests.test_resident import POOL, same, spec, start
 
 pytestmark = pytest.mark.gpu
 
@@ -66,6 +66,33 @@ def test_later_launches_do_not_wait(gpu):
         d.Step(1e-5, 500)
         d.Synchronize()
     assert time.perf_counter() - t < 5.0  # a wait takes 20 s
+
+
+@pytest.mark.parametrize("box", [False, True])
+def test_reset_makes_the_handle_usable_again(gpu, box):
+    out = []
+    for fail in (True, False):
+        sp, d = boxed() if box else plain()
+        dt = sp.meta["dt_ms"]
+        if fail:
+            for _ in range(2):  # the second time after a whole run
+                give_up(d, dt)
+                with GAVE_UP:
+                    d.Synchronize()
+                d.Reset()
+                d.InitOpeningAll()
+                d.UpdatePools() if box else d.Update(*sp.rim_arrays(), sp.jsr_array([1000.0]))
+                d.Step(dt, 100)
+                d.Synchronize()
+            d.Reset()
+            d.InitOpeningAll()
+            d.UpdatePools() if box else d.Update(*sp.rim_arrays(), sp.jsr_array([1000.0]))
+        for k in (50, 100, 350):
+            d.Step(dt, k)
+        out.append([d.GetField(f) for f in range(sp.n_ions + sp.n_bound)] +
+                   [d.GetChannelsStates(), d.GetRngStates(), d.GetTotalSRCurrent(), d.GetReleaseStats()] +
+                   ([d.GetCytosolBox(f) for f in range(d.CytosolBoxFields())] if box else []))
+    same(*out)
 
 
 def test_limit_is_checked(gpu):
