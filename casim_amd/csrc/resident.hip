@@ -138,11 +138,10 @@ __device__ __forceinline__ bool flags_out(const unsigned *watch, unsigned target
     return !__ballot(watch && (int)(xld(watch) - target) < 0);
 }
 // Wait for them; false when the limit has passed, which only a missing partner
-// workgroup could cause.  A limit of 0: not at all.
+// workgroup could cause.
 __device__ __forceinline__ bool wait_flags(const unsigned *watch, unsigned target, long long limit) {
     long long t0 = 0;
     for (unsigned n = 1; !flags_out(watch, target); ++n) {
-        if (limit == 0) return false;
         if ((n & 255u) == 0) {
             const long long t = wall_clock64();
             if (!t0) t0 = t;
@@ -705,7 +704,7 @@ __global__ __launch_bounds__(64 * res_waves(PS), (res_waves(PS) + 3) / 4) void k
         int bin_in = r.trace ? (int)(r.trace_every - m0 % r.trace_every) : 0;
         long long bin = r.trace ? m0 / r.trace_every + 1 : 0;
         __syncthreads();  // map complete
-        bool ok = true;
+        bool ok = r.limit != 0 || r.G == 1;  // without a limit to wait, give up right away
         int pos = n;     // draws of the last step
         int stale = 0;   // 1: the other copy of pg misses the last step's toggles
         // streams and draws of the next step

@@ -361,8 +361,8 @@ int casim_dyad_set_split(CasimDyad *d, int32_t on);
  * the reference).  Only something else that holds the GPU's compute units could
  * make it wait that long; then the launch gives up, launches behind it leave at
  * once, and every call that waits for the handle's stream, and casim_dyad_step,
- * returns CASIM_E_DEVICE: the state is invalid until casim_dyad_reset.  0: no
- * wait at all, so that nearly every such step gives up. */
+ * returns CASIM_E_DEVICE: the state is invalid until casim_dyad_reset.  0: a
+ * launch with several workgroups per site gives up right away. */
 int casim_dyad_set_wait_limit(CasimDyad *d, double seconds);
 
 /*

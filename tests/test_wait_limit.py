@@ -1,6 +1,6 @@
-"""A step whose workgroups may not wait for each other gives up: every kernel
-ends as usual, every call says that the state is invalid, and no later launch of
-the handle waits for workgroups that have left."""
+"""A step whose workgroups may not wait for each other gives up right away: every
+kernel ends as usual, every call says that the state is invalid, and no later
+launch of the handle waits for workgroups that have left."""
 import time
 
 import numpy as np
