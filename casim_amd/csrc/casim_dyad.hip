@@ -166,6 +166,12 @@ bool CasimDyad::pair_ok() const {
     if (steps_per_pass < 2 || !use_sweep || sweep_threads <= 0 || (Q.on && Q.cyto)) return false;
     // a cytosol box steps between passes only with an even number of substeps
     if (box && casim::box_substeps(this) % 2 != 0) return false;
+    // Species read at run time (see sweep2_species) with more than two nodes per
+    // thread: the pair pass would spill a thousand registers, some of them in front
+    // of a lane mask's restore, and was slower (FP32, us per step, pairs and one
+    // step per pass: 512 sites of 61x600 5833 and 1818, of 81x121x5 6363 and 5525).
+    const bool known = layout_id(P) || (P.ni == 2 && P.nb == 4 && P.n_grid == 6 && P.n_face == 0);
+    if (!known && P.ny * P.nz > 2 * sweep_threads) return false;
     return 4 * (size_t)P.n_grid * P.ny * P.nz * tsize <= 64 * 1024;
 }
 

@@ -67,8 +67,9 @@ void sweep2_slots(CasimDyad *d, double dt) {
     const int P = d->P.ny * d->P.nz;
     const int sl = (P + d->sweep_threads - 1) / d->sweep_threads;
     if (sl <= 1) return sweep2_launch<T, DIM, NI, NB, NG, NF, LY, 1>(d, dt);
-    if (sl <= 2) return sweep2_launch<T, DIM, NI, NB, NG, NF, LY, 2>(d, dt);
-    return sweep2_launch<T, DIM, NI, NB, NG, NF, LY, 4>(d, dt);
+    if constexpr (NI != 0)  // run-time species: see CasimDyad::pair_ok
+        if (sl > 2) return sweep2_launch<T, DIM, NI, NB, NG, NF, LY, 4>(d, dt);
+    return sweep2_launch<T, DIM, NI, NB, NG, NF, LY, 2>(d, dt);
 }
 
 template <typename T, int DIM>

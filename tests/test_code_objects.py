@@ -1,4 +1,4 @@
-"""The machine code of the kernels that hold a site's state over many steps.
+"""The machine code of the built kernels.
 
 Where a vector register is spilled just before a lane mask is widened again, the
 lanes outside the mask lose its value; the compiler has done that to registers
@@ -15,7 +15,6 @@ from casim_amd import abi
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 WRITES = re.compile(r"v_(?!cmp|readlane|readfirstlane)|ds_read|ds_bpermute|(global|flat|scratch|buffer)_load")
-ENDS = re.compile(r"s_cbranch|s_branch|s_endpgm|s_setpc")
 
 
 def registers(text):
@@ -35,10 +34,12 @@ def slot(ins):
     return re.search(r"offset:(\d+)|$", ins).group(1) or "0"
 
 
-def lost_spills(code):
+def lost_spills(code, before=None):
     """Spill stores right before an exec mask is restored, of registers that
     nothing has written since the mask was saved, into slots that no other
-    store fills and a load outside the mask reads."""
+    store fills and a load outside the mask reads.  before: the instructions
+    that may run before each one (by default the one above it)."""
+    before = before or [[i - 1] if i else [] for i in range(len(code))]
     stores, loads = {}, {}
     for i, ins in enumerate(code):
         if ins.startswith("scratch_store"):
@@ -50,22 +51,32 @@ def lost_spills(code):
         m = re.match(r"s_or_b64 exec, exec, (s\[\d+:\d+\])", ins)
         if not m:
             continue
-        save = j = i - 1
-        while save > 0 and not re.match(r"s_\w*saveexec_b64 " + re.escape(m.group(1)) + r",", code[save]):
-            save -= 1
-        while j > save and not ENDS.match(code[j]):
-            k, j = j, j - 1
-            if not code[k].startswith("scratch_store") or stores[slot(code[k])] != [k]:
-                continue
-            if not any(not save < n < i for n in loads.get(slot(code[k]), [])):
-                continue
-            if registers(code[k]) - set().union(*(written(c) for c in code[save:k])):
-                bad.insert(0, code[k])
+        k, late = i - 1, []
+        while k >= 0 and not code[k].startswith(("s_branch", "s_cbranch", "s_endpgm")) and \
+                not re.search(r"\bexec\b|saveexec", code[k].partition(",")[0]):
+            if code[k].startswith("scratch_store") and stores[slot(code[k])] == [k]:
+                late.append(k)
+            k -= 1
+        if not late:
+            continue
+        # what runs under the mask: everything from its save to here
+        save = re.compile(r"s_\w*saveexec_b64 " + re.escape(m.group(1)) + ",")
+        masked, todo = set(), list(before[i])
+        while todo:
+            n = todo.pop()
+            if n not in masked and not save.match(code[n]):
+                masked.add(n)
+                todo += before[n]
+        since = set().union(*(written(code[n]) for n in masked))
+        for k in reversed(late):
+            if registers(code[k]) - since and any(n not in masked for n in loads.get(slot(code[k]), [])):
+                bad.append(code[k])
     return bad
 
 
 def kernels(tmp_path):
-    """(name, instructions) of every kernel in the built library."""
+    """(name, instructions, what may run before each) of every kernel in the
+    built library that spills vector registers."""
     lib = shutil.copy(abi.LIB_PATH, tmp_path / "lib.so")
     subprocess.run([OBJDUMP, "--offloading", lib], check=True, capture_output=True, cwd=tmp_path)
     for f in sorted(os.listdir(tmp_path)):
@@ -75,7 +86,20 @@ def kernels(tmp_path):
                               text=True).stdout
         for part in re.split(r"\n[0-9a-f]+ <", text)[1:]:
             name, _, body = part.partition(">:\n")
-            yield name, [line.split("//")[0].strip() for line in body.split("\n") if line.startswith("\t")]
+            if "scratch_store" not in body:
+                continue
+            lines = [line.split("//") for line in body.split("\n") if line.startswith("\t") and "//" in line]
+            code = [a.strip() for a, _ in lines]
+            at = {int(b.split(":")[0], 16): i for i, (_, b) in enumerate(lines)}
+            start = min(at)
+            before = [[] for _ in code]
+            for i, ins in enumerate(code):
+                target = re.search(r"\+0x([0-9a-f]+)>", lines[i][1])
+                if ins.startswith(("s_branch", "s_cbranch")):
+                    before[at[start + int(target.group(1), 16)] if target else 0].append(i)
+                if not ins.startswith(("s_branch", "s_endpgm")) and i + 1 < len(code):
+                    before[i + 1].append(i)
+            yield name, code, before
 
 
 def test_lost_spills_are_found():
@@ -91,10 +115,9 @@ def test_lost_spills_are_found():
 
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
-def test_no_spill_is_lost_in_the_step_kernels(tmp_path):
+def test_no_spill_is_lost(tmp_path):
     names = []
-    for name, code in kernels(tmp_path):
-        if re.search(r"k_resident|k_site2d", name):
-            names.append(name)
-            assert lost_spills(code) == [], name
-    assert len(names) >= 20
+    for name, code, before in kernels(tmp_path):
+        names.append(name)
+        assert lost_spills(code, before) == [], name
+    assert names
