@@ -1520,8 +1520,9 @@ int casim_mlp_predict(CasimMLP *m, const float *x, int64_t rows, float *mean, fl
         m->predict_reserve(chunk);
         // two slots: while a chunk is evaluated, the next one is copied to pinned
         // memory and on to the device, and the outputs, which the kernel writes to
-        // pinned memory, go to the caller (five members, us: 55003 rows 530, 740 with
-        // one copy each from and to pageable memory; 100 rows 39, 150)
+        // pinned memory, go to the caller (five members, us: 55003 rows 530, 690 where
+        // every call brings an array that was not used before, 740 and more with one
+        // copy each from and to pageable memory; 100 rows 39, 150)
         const int cap = m->pr_rows, nc = (int)((rows + chunk - 1) / chunk);
         const size_t slot = (size_t)cap * (m->n_in + E + 2);
         auto take = [&](int c) {

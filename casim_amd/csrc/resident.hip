@@ -19,21 +19,33 @@
 // together and a waiting slab's partners have started or will start when
 // earlier sites end.
 //
-// What bounds it: the row of barriers.  At 20 planes of doubles a step takes
-// 9.0 us on every CU, of which FP64 issue of the fullest SIMD is 5 us; with
-// phases of four planes (9.4 us) the barriers and the channel wave alone took
-// 6.4 us.  In FP32 40 planes take 12 us, 10 us of them issue.  Fewer
-// planes per slab finish a step sooner, more planes carry more sites at once.
-// Measured (81x81x5, us per step; k_sweep2 with the channel kernels before):
+// What bounds it: phases that do one thing at a time.  At 20 planes of doubles
+// a step takes 8.8 us on every CU: 2420 vector instructions per SIMD (4.0 us)
+// and 2300 LDS instructions per CU (3.8 us), which two waves per SIMD between
+// barriers hardly overlap.  In FP32 40 planes take 12 us, 10 us of them vector
+// issue.  Fewer planes per slab finish a step sooner, more planes carry more
+// sites at once.
+// Measured (81x81x5, us per step in calls of 2000 steps, 200 for 1024 and 4096
+// sites; shorter calls share the load and write-out of the state among fewer
+// steps; k_sweep2 with the channel kernels before):
 //   sites   FP64 k_sweep2   FP64 here   FP32 k_sweep2   FP32 here
-//       1        98             4.2           -             -
-//       6        99             4.3           -             3.7
-//      32       106             6.8           -             -
-//    1024         -           144             -            98
-//    4096       780           572           440           392
-// More workgroups per CU (128 registers each) took 765 and 362; two planes at a
-// time 604; waves waiting for their neighbour waves by LDS counters in place of
-// barriers 919 and more.
+//       1        98             3.5           -             2.9
+//       6        99             3.5           -             2.9
+//      32       106             5.6           -             4.2
+//    1024         -           139             -            96
+//    4096       780           554           440           379
+// At 4096 sites in FP64, when a step here took 572 us: two planes at a time
+// 604; waves waiting for their neighbour waves by LDS counters in place of
+// barriers 919 and more; two workgroups per CU with 128 registers each 765.
+// In FP32 those two workgroups took 362 us against 392; they are not built,
+// because a variant of that arrangement ended in an illegal memory access whose
+// cause was not shown.
+// A register spilled in a divergent block must not be read after the lanes meet
+// again: this compiler places the store of such a spill in front of the mask
+// that brings the other lanes back, which lose the value.  The channel wave's
+// shared stores are therefore made by all lanes, the file is built without the
+// hoisting of constants that caused most spills, and tests/test_code_objects.py
+// reads the built code for it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -918,7 +930,9 @@ Form form(double us0, double us1) {
             launch_form<T, PL, PH, PS, FLAT>};
 }
 const Form FORMS[] = {
-    // fewer phases as LDS allows: six planes each fit up to 408 nodes (4096 sites: 572 us per step, 599 with four)
+    // six planes a phase, built for up to 408 nodes (4096 sites: 572 us per step when four took 599); four up to 440,
+    // though LDS would hold six there.  G slabs of 20 planes take nx - 2 from 17 G to 20 G; the widths between (61 to
+    // 67, 81 to 84) fall to 10 planes, which gain little over the sweeps in large batches.
     form<double, 20, 6, 408>(2.1, 0.343), form<double, 20, 4, 440>(2.1, 0.37), form<double, 10, 3, 440>(2.1, 0.37),
     form<double, 5, 3, 440>(2.1, 0.37),
     form<float, 40, 8, 440>(2.0, 0.25),  form<float, 20, 6, 440>(2.0, 0.25),  form<float, 10, 3, 440>(2.0, 0.25),

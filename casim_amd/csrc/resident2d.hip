@@ -67,7 +67,7 @@ struct PlaneNbr {
 // (node_update), k_channels, k_efflux, pool_update_site, pool_advance_site and
 // k_rim in their order, so the values are the same bits.
 // What bounds it: the slowest of the three roles between the barriers (100 sites
-// of 31 x 41 nodes with two ions and every compartment: 7.0 us per step, 9.1
+// of 31 x 41 nodes with two ions and every compartment: 7.2 us per step, 9.1
 // with the species layout read at run time, 6.6 without the grid update; four
 // launches of 107 us together before).  A site's state does not leave the CU
 // and there is no launch per step, so any number of steps and sites gains.
